@@ -7,14 +7,15 @@
 //   router        r = W_router @ x (float32), 16 experts of one token per
 //                 workgroup (router_logits); then p = softmax(r), top-k by p
 //                 with ties to the lower expert id (one wave per token, lane =
-//                 expert) and the plan, in one workgroup (topk_plan)
-//   route_plan    groups the (token, expert) pairs by expert: routed experts in
-//                 id order, then the shared experts (every token, weight 1)
+//                 expert)
+//   plan          groups the (token, expert) pairs by expert, in one workgroup
+//                 (with the top-k for small batches): the shared experts
+//                 (every token, weight 1) and the routed experts in id order,
+//                 in groups of at most 64 rows
 //   expert GEMMs  gate/up + SwiGLU, then down, each expert's weights streamed
-//                 once for all of its tokens: up to 16 rows per expert on
-//                 expert_slab (one workgroup per 16 outputs of an expert, K
-//                 split over its waves, every weight fragment requested at
-//                 once); more rows on prefill.hip's grouped GEMM
+//                 once per group (expert_slab: one workgroup per 16 or 32
+//                 outputs of a group, K split over its waves, the weights
+//                 read from MFMA-native copies)
 //   combine       y = bf16(sum_k p_k * e_k + sum_s e_s) in float32, rank order,
 //                 one thread per output element
 // Rounding points follow the dense layer: bf16 after gate/up, after SwiGLU and
@@ -51,8 +52,10 @@ constexpr int kMaxShared = 8;
 constexpr int kMaxTopK = 16;
 
 constexpr int kRouterRows = 16;  // routed experts per router_logits workgroup
-constexpr int kPlanThreads = 1024;  // topk_plan: one wave per token, 16 at a time
+constexpr int kPlanThreads = 1024;
+constexpr int kPlanTokens = kPlanThreads / 64;  // topk_plan: one wave per token
 constexpr int kMaxTokens = 256;
+constexpr int kMaxPairWords = kMaxTokens * kMaxTopK / 64;
 
 // r[t][e] = W_router[e] . x[t] in float32 for the kRouterRows experts e0.. of
 // token t = blockIdx.x: wave w takes experts e0 + 4 w .. + 3 and requests
@@ -103,6 +106,19 @@ __global__ __launch_bounds__(kThreads) void router_logits_kernel(const uint16_t*
   }
 }
 
+// The largest of the wave's 64 values in every lane (DPP row moves, then the
+// last lane's value: a few cycles per step, where a shuffle goes through LDS).
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+  auto step = [&](uint32_t w) { v = max(v, w); };
+  step(__builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
+  step(__builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false));   // quad_perm 2,3,0,1
+  step(__builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+  step(__builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false));  // row_mirror
+  step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast15 into rows 1 and 3
+  step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0x8, 0xf, false));  // row_bcast31 into row 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // p = softmax(r) over the routed experts and the top K by p (ties to the
 // lower expert id) of token t, on one wave (lane = expert).
 __device__ __forceinline__ void topk_wave(const float* logits, int t, int E, int K, int lane, int32_t* ids,
@@ -113,150 +129,139 @@ __device__ __forceinline__ void topk_wave(const float* logits, int t, int E, int
   const float ex = live ? expf(r - m) : 0.0f;
   const float s = group_sum<64>(ex);
   const float p = ex / s;
-  bool alive = live;
+  // an order-preserving key per lane, never zero; the lowest lane that holds
+  // the largest key is the expert that argmax over (p, -id) gives
+  uint32_t key = live ? (uint32_t)(argmax_key(p, 0) >> 32) : 0u;
+  int mine = 0;
+  float pmine = 0.0f;
   for (int k = 0; k < K; ++k) {
-    unsigned long long key = alive ? argmax_key(p, (uint32_t)lane) : 0ull;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) key = umax64(key, shfl_xor_u64(key, off));
-    const int idx = (int)argmax_key_index(key);
-    const float pw = __shfl(p, idx, 64);
-    if (lane == 0) {
-      ids[t * K + k] = idx;
-      weights[t * K + k] = pw;
-      ids_lds[t * K + k] = idx;
-    }
-    if (lane == idx) alive = false;
+    const int idx = __ffsll(__ballot(key == wave_umax(key))) - 1;
+    const float pw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), idx));
+    if (lane == k) mine = idx, pmine = pw;
+    if (lane == idx) key = 0u;
+  }
+  if (lane < K) {
+    ids[t * K + lane] = mine;
+    weights[t * K + lane] = pmine;
+    if (ids_lds) ids_lds[t * K + lane] = mine;
   }
 }
+
+// One launch entry of the expert GEMMs: at most kGroupRows rows of an expert,
+// rows 0 for an entry past the last.
+struct ExpertGroup {
+  int expert, offset, rows, unused;
+};
+constexpr int kGroupRows = 64;
+
+struct PlanLds {
+  unsigned long long bits[kMaxRouted][kMaxPairWords];  // expert e's pairs, one bit each
+  uint16_t before[kMaxRouted][kMaxPairWords];          // its pairs before word w
+  int32_t ids[kMaxTokens * kMaxTopK];
+  int counts[kMaxRouted];
+  int offs[kMaxRouted + kMaxShared];
+  int n_groups;
+};
 
 // The grouping of the T*(K+S) (token, expert) pairs by expert, from the ids
-// in LDS, on the calling workgroup (nt threads; every thread calls it):
-// counts by LDS atomics; the offsets and the non-empty groups on wave 0 (lane
-// e: routed expert e, a prefix sum across lanes, the group index from a
-// ballot; the shared experts follow the routed pairs); then routed expert
-// e's slots by thread e, which walks the pairs in token order (an expert
-// appears at most once per token from the router; repeated caller ids take
-// consecutive slots), and shared expert s's slots (one per token) by thread
-// E + s.  Within an expert the slots follow token order, so the plan does not
-// depend on timing.
-// `tokens` (distinct: every token names an expert at most once, T <= 64):
-// routed expert e's tokens as a bit mask, and pair (t, k)'s slot is e's
-// offset plus the number of e's tokens before t, all pairs at once.
-__device__ void plan_pairs(const int32_t* ids, int T, int K, int E, int S, int nt, int* counts, int* offs,
-                           unsigned long long* tokens, bool distinct, int32_t* grp_expert, int32_t* grp_count,
-                           int32_t* grp_offset, int32_t* n_groups, int32_t* a_rows, int32_t* pair_slot) {
-  static_assert(kMaxRouted <= 64, "one lane per routed expert");
-  const int tid = threadIdx.x;
-  const int total = E + S, per = K + S;
-  auto clamp = [&](int e) { return e < 0 ? 0 : (e >= E ? E - 1 : e); };
-  distinct = distinct && T <= 64;
-  for (int e = tid; e < E; e += nt) {
-    counts[e] = 0;
-    tokens[e] = 0ull;
-  }
+// in LDS, on the calling workgroup (every thread calls it): pair i = t K + k
+// sets bit i of its expert's mask, and its slot is the expert's offset plus
+// the number of the expert's pairs before it (the popcounts of the whole
+// words before its own, from a prefix sum per expert, and of the word's lower
+// bits), so the slots follow pair order whatever the timing and an expert may
+// appear twice for a token.  A serial walk over the pairs by one thread per
+// expert had taken 200 us of a 256-token call; the masks take about 4.  The
+// groups list the shared experts first (every token: the longest), then the
+// non-empty routed ones in id order, in runs of at most kGroupRows rows; the
+// slots list the routed pairs by expert, then the shared experts' rows.
+__device__ void plan_pairs(PlanLds& l, int T, int K, int E, int S, int max_groups, ExpertGroup* groups,
+                           int32_t* a_rows, int32_t* pair_slot) {
+  static_assert(kMaxRouted <= 64 && kMaxPairWords <= 64, "one lane per routed expert and per word of pairs");
+  const int tid = threadIdx.x, nt = blockDim.x, wave = tid >> 6, lane = tid & 63;
+  const int P = T * K, W = (P + 63) / 64, per = K + S;
+  auto expert_of = [&](int i) { return min(max(l.ids[i], 0), E - 1); };
+  for (int i = tid; i < E * W; i += nt) l.bits[i / W][i % W] = 0ull;
   __syncthreads();
-  for (int i = tid; i < T * K; i += nt) {
-    const int e = clamp(ids[i]);
-    atomicAdd(&counts[e], 1);
-    if (distinct) atomicOr(&tokens[e], 1ull << (i / K));
-  }
+  for (int i = tid; i < P; i += nt) atomicOr(&l.bits[expert_of(i)][i >> 6], 1ull << (i & 63));
   __syncthreads();
-  if (tid < 64) {
-    const int lane = tid;
-    const int c = lane < E ? counts[lane] : 0;
-    int incl = c;
+  auto inclusive = [&](int v) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
+      const int up = __shfl_up(v, d, 64);
+      if (lane >= d) v += up;
     }
-    const unsigned long long nonempty = __ballot(c > 0);
-    const int g = __popcll(nonempty & ((1ull << lane) - 1ull));
-    const int nr = __popcll(nonempty);
+    return v;
+  };
+  for (int e = wave; e < E; e += nt / 64) {
+    const int c = lane < W ? __popcll(l.bits[e][lane]) : 0;
+    const int incl = inclusive(c);
+    if (lane < W) l.before[e][lane] = (uint16_t)(incl - c);
+    if (lane == 63) l.counts[e] = incl;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int shared_runs = (T + kGroupRows - 1) / kGroupRows;
+    const int c = lane < E ? l.counts[lane] : 0, runs = (c + kGroupRows - 1) / kGroupRows;
+    const int off = inclusive(c) - c, last_run = inclusive(runs), first = S * shared_runs + last_run - runs;
     if (lane < E) {
-      offs[lane] = incl - c;
-      if (c > 0) {
-        grp_expert[g] = lane;
-        grp_count[g] = c;
-        grp_offset[g] = incl - c;
-      }
+      l.offs[lane] = off;
+      for (int j = 0; j < runs; ++j)
+        groups[first + j] = {lane, off + j * kGroupRows, min(kGroupRows, c - j * kGroupRows), 0};
     }
-    if (lane < S) {  // shared expert lane: every token, after the routed pairs
-      offs[E + lane] = T * K + lane * T;
-      grp_expert[nr + lane] = E + lane;
-      grp_count[nr + lane] = T;
-      grp_offset[nr + lane] = T * K + lane * T;
+    if (lane < S) {
+      const int so = P + lane * T;
+      l.offs[E + lane] = so;
+      for (int j = 0; j < shared_runs; ++j)
+        groups[lane * shared_runs + j] = {E + lane, so + j * kGroupRows, min(kGroupRows, T - j * kGroupRows), 0};
     }
-    if (lane == 0) *n_groups = nr + S;
+    if (lane == 63) l.n_groups = S * shared_runs + last_run;
   }
   __syncthreads();
-  if (distinct) {
-    for (int i = tid; i < T * (K + S); i += nt) {
-      const int t = i / per, k = i % per;
-      int slot;
-      if (k < K) {
-        const int e = clamp(ids[t * K + k]);
-        slot = offs[e] + __popcll(tokens[e] & ((1ull << t) - 1ull));
-      } else {
-        slot = offs[E + k - K] + t;
-      }
-      a_rows[slot] = t;
-      pair_slot[t * per + k] = slot;
-    }
-    return;
-  }
-  for (int e = tid; e < total; e += nt) {
-    int slot = offs[e];
-    if (e < E) {
-#pragma unroll 8
-      for (int i = 0; i < T * K; ++i)
-        if (clamp(ids[i]) == e) {
-          a_rows[slot] = i / K;
-          pair_slot[(i / K) * per + i % K] = slot;
-          ++slot;
-        }
+  for (int i = l.n_groups + tid; i < max_groups; i += nt) groups[i] = {0, 0, 0, 0};
+  for (int i = tid; i < T * per; i += nt) {
+    const int t = i / per, k = i % per;
+    int slot;
+    if (k < K) {
+      const int pair = t * K + k, e = expert_of(pair), w = pair >> 6;
+      slot = l.offs[e] + l.before[e][w] + __popcll(l.bits[e][w] & ((1ull << (pair & 63)) - 1ull));
     } else {
-      for (int t = 0; t < T; ++t, ++slot) {
-        a_rows[slot] = t;
-        pair_slot[t * per + K + (e - E)] = slot;
-      }
+      slot = l.offs[E + k - K] + t;
     }
+    a_rows[slot] = t;
+    pair_slot[t * per + k] = slot;
   }
 }
 
-// Top-k of every token (wave w takes tokens w, w + 16, ...), then the plan.
+// Top-k of every token (one wave each) and the plan, one workgroup: batches
+// of up to kPlanTokens tokens, one token per wave.
 __global__ __launch_bounds__(kPlanThreads) void topk_plan_kernel(const float* logits, int T, int E, int K, int S,
-                                                                 int32_t* ids, float* weights, int32_t* grp_expert,
-                                                                 int32_t* grp_count, int32_t* grp_offset,
-                                                                 int32_t* n_groups, int32_t* a_rows,
+                                                                 int max_groups, int32_t* ids, float* weights,
+                                                                 ExpertGroup* groups, int32_t* a_rows,
                                                                  int32_t* pair_slot) {
-  __shared__ int32_t sids[kMaxTokens * kMaxTopK];
-  __shared__ int counts[kMaxRouted + kMaxShared];
-  __shared__ int offs[kMaxRouted + kMaxShared];
-  __shared__ unsigned long long tokens[kMaxRouted];
+  __shared__ PlanLds l;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int t = wave; t < T; t += kPlanThreads / 64) topk_wave(logits, t, E, K, lane, ids, weights, sids);
+  if (wave < T) topk_wave(logits, wave, E, K, lane, ids, weights, l.ids);
   __syncthreads();
-  // (the top-k of a token names each expert once)
-  plan_pairs(sids, T, K, E, S, kPlanThreads, counts, offs, tokens, true, grp_expert, grp_count, grp_offset,
-             n_groups, a_rows, pair_slot);
+  plan_pairs(l, T, K, E, S, max_groups, groups, a_rows, pair_slot);
 }
 
-// The plan for caller-supplied ids (hk_moe_experts): the ids are copied to
-// LDS, then grouped.
-__global__ __launch_bounds__(kThreads) void route_plan_kernel(const int32_t* ids, int T, int K, int E, int S,
-                                                              int32_t* grp_expert, int32_t* grp_count,
-                                                              int32_t* grp_offset, int32_t* n_groups,
-                                                              int32_t* a_rows, int32_t* pair_slot) {
-  __shared__ int32_t sids[kMaxTokens * kMaxTopK];
-  __shared__ int counts[kMaxRouted + kMaxShared];
-  __shared__ int offs[kMaxRouted + kMaxShared];
-  __shared__ unsigned long long tokens[kMaxRouted];
-  for (int i = threadIdx.x; i < T * K; i += kThreads) sids[i] = ids[i];
+// Top-k alone, for larger batches: one wave per token over many workgroups
+// (16 tokens after each other on each wave of one workgroup took 35 us of a
+// 256-token call).
+__global__ __launch_bounds__(kThreads) void topk_kernel(const float* logits, int T, int E, int K, int32_t* ids,
+                                                        float* weights) {
+  const int t = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (t < T) topk_wave(logits, t, E, K, threadIdx.x & 63, ids, weights, nullptr);
+}
+
+// The plan alone: ids from topk_kernel or the caller.
+__global__ __launch_bounds__(kPlanThreads) void route_plan_kernel(const int32_t* ids, int T, int K, int E, int S,
+                                                                  int max_groups, ExpertGroup* groups,
+                                                                  int32_t* a_rows, int32_t* pair_slot) {
+  __shared__ PlanLds l;
+  for (int i = threadIdx.x; i < T * K; i += kPlanThreads) l.ids[i] = ids[i];
   __syncthreads();
-  // (caller ids may name an expert twice for one token: the serial slots)
-  plan_pairs(sids, T, K, E, S, kThreads, counts, offs, tokens, false, grp_expert, grp_count, grp_offset, n_groups,
-             a_rows, pair_slot);
+  plan_pairs(l, T, K, E, S, max_groups, groups, a_rows, pair_slot);
 }
 
 // y[t][d] = bf16(sum_k p_k e_k[d] + sum_s e_s[d]) in float32, ranks in order;
@@ -284,97 +289,170 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
   return (g / (1.0f + expf(-clipped))) * u;
 }
 
-constexpr int kSlabThreads = 512;               // expert_slab: 8 waves
-constexpr int kSlabWavesE = kSlabThreads / 64;
-constexpr int kSlabBatchE = 8;                  // K steps per wave requested at once
-constexpr int kSlabMaxRowsE = 16;               // rows per expert group on expert_slab
+struct ExpertGemmArgs {
+  const uint16_t* A;          // row-major bf16 rows of K values
+  const uint16_t* Wn;         // MFMA-native copies of the experts' weights, w_stride apart
+  uint16_t* Y;                // [slots, N]
+  const ExpertGroup* groups;  // gridDim.y entries
+  const int32_t* a_rows;      // A row of each slot (PAIR; else the slot itself)
+  long long w_stride;
+  int N, K, a_bytes;          // bytes of A
+};
 
-// Expert GEMM for groups of at most 16 rows (the decode batch).  Workgroup
-// (s, z) computes outputs 16 s .. + 15 of group z's expert (the MFMA-native
-// copy Wn + expert * w_stride) for the group's rows: wave w takes the 32-column K steps w, w +
-// 8, ..., requests the weight fragments (and the up rows' for SwiGLU) and the
-// row fragments of up to kSlabBatchE of them at once, and multiplies on MFMA
-// 16x16x32 (rows x outputs); the waves' partial sums meet in LDS and are added
-// in wave order.  Row i of the group reads A row a_rows[offset + i] (or offset
-// + i) and writes output row offset + i.  Epilogue as the dense layer:
-// SwiGLU bf16(silu(bf16(g)) * bf16(u)), else bf16.
-// TWO (without SwiGLU): the workgroup takes outputs 32 s .. + 31, the second
-// 16 in place of the up rows (one row fragment, two weight fragments per K step).
-template <bool PAIR, bool TWO = false>
-__global__ __launch_bounds__(kSlabThreads) void expert_slab_kernel(PrefillGemmArgs a) {
-  static_assert(!(PAIR && TWO), "SwiGLU pairs take one slab");
-  constexpr bool U = PAIR || TWO;  // a second weight fragment per step
-  __shared__ f32x4 red[U ? 2 : 1][kSlabWavesE][64];
-  const int z = blockIdx.y;
-  if (z >= *a.n_groups) return;
-  const int count = min(a.grp_count[z], kSlabMaxRowsE);
-  const int off = a.grp_offset[z];
-  const int n0 = blockIdx.x * (TWO ? 32 : 16);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// The outputs n0 .. of one group on RB blocks of 16 rows, NF weight fragments
+// of 16 weight rows per K step (PAIR: NF / 2 gate and NF / 2 up ones); see
+// expert_slab_kernel.
+template <bool PAIR, int NF, int WAVES, int RB, int DEPTH>
+__device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const ExpertGroup& g, int n0, f32x4* red) {
+  constexpr int NO = PAIR ? NF / 2 : NF;  // 16-output blocks
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fk = (lane >> 4) * 8;
   const int N = a.N, K = a.K;
-  // the expert's MFMA-native copy (Wn: [rows / 16][K / 8][16] pieces of 8
-  // weights, a fragment's 16 rows one 256-byte run, a wave's K step one 1 KiB
-  // run)
-  const uint16_t* W = static_cast<const uint16_t*>(a.Wn) + (size_t)a.grp_expert[z] * (size_t)a.w_stride;
-  const __amdgpu_buffer_rsrc_t wr = rsrc(W, (PAIR ? 2 : 1) * N * K * 2);
-  // this lane's piece of its weight row (and up row) and its A row at column
-  // fk; rows past the ends read zero
-  auto piece = [&](int n) { return (unsigned)((((n >> 4) * (K >> 3) + (fk >> 3)) * 16 + (n & 15)) * 16); };
-  const unsigned wofs = n0 + fr < N ? piece(n0 + fr) : 0x7ffffff0u;
-  const unsigned uofs = PAIR ? (n0 + fr < N ? piece(N + n0 + fr) : 0x7ffffff0u)
-                             : (n0 + 16 + fr < N ? piece(n0 + 16 + fr) : 0x7ffffff0u);
-  const int arow = fr < count ? (a.a_rows ? a.a_rows[off + fr] : off + fr) : -1;
-  const __amdgpu_buffer_rsrc_t ar = rsrc(a.A + (size_t)(arow < 0 ? 0 : arow) * a.lda, arow < 0 ? 0 : K * 2);
-  const unsigned aofs = (unsigned)fk * 2u;
+  // Wn of an expert: [rows / 16][K / 8][16] pieces of 8 weights, so a
+  // fragment's 16 rows are one 256-byte run and a wave's K step one 1 KiB run
+  const __amdgpu_buffer_rsrc_t wr = rsrc(a.Wn + (size_t)g.expert * (size_t)a.w_stride, (PAIR ? 2 : 1) * N * K * 2);
+  const __amdgpu_buffer_rsrc_t ar = rsrc(a.A, a.a_bytes);
+  // this lane's piece of its weight row in each fragment, and the numbers of
+  // its A rows; outputs and rows past the ends read zero
+  constexpr unsigned kOutside = 0x7ffffff0u;
+  unsigned wofs[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int n = n0 + 16 * (f % NO) + fr, r = f < NO ? n : N + n;
+    wofs[f] = n < N ? (unsigned)((((r >> 4) * (K >> 3) + (fk >> 3)) * 16 + (r & 15)) * 16) : kOutside;
+  }
+  const __amdgpu_buffer_rsrc_t rr = rsrc(PAIR ? a.a_rows + g.offset : nullptr, PAIR ? g.rows * 4 : 0);
+  unsigned row[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+    row[b] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(rr, (16 * b + fr) * 4, 0, 0) : g.offset + 16 * b + fr;
   const int steps = K / 32;
-  const int mine = steps > wave ? (steps - wave + kSlabWavesE - 1) / kSlabWavesE : 0;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, accu = {0.f, 0.f, 0.f, 0.f};
-  for (int j0 = 0; j0 < mine; j0 += kSlabBatchE) {
-    u32x4 w[kSlabBatchE], u[U ? kSlabBatchE : 1], x[kSlabBatchE];
+  const int mine = steps > wave ? (steps - wave + WAVES - 1) / WAVES : 0;
+  f32x4 acc[RB][NF];
 #pragma unroll
-    for (int i = 0; i < kSlabBatchE; ++i) {
-      const bool live = j0 + i < mine;
-      const int st = wave + kSlabWavesE * (j0 + i);
-      const unsigned k0b = (unsigned)(32 * st) * 2u;  // bytes along an A row
-      const unsigned k0w = (unsigned)st * 4u * 256u;  // four k groups of 16 pieces in the native copy
-      w[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, live ? wofs + k0w : 0x7ffffff0u, 0, 2);
-      if constexpr (U) u[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, live ? uofs + k0w : 0x7ffffff0u, 0, 2);
-      x[i] = __builtin_amdgcn_raw_buffer_load_b128(ar, live ? aofs + k0b : 0x7ffffff0u, 0, 0);
-    }
+  for (int b = 0; b < RB; ++b)
 #pragma unroll
-    for (int i = 0; i < kSlabBatchE; ++i) {
-      const bf16x8 xa = __builtin_bit_cast(bf16x8, x[i]);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8, w[i]), acc, 0, 0, 0);
-      if constexpr (U)
-        accu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8, u[i]), accu, 0, 0, 0);
+    for (int f = 0; f < NF; ++f) acc[b][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a ring of DEPTH K steps per wave: a step's products free its slot for the
+  // loads of the step DEPTH on, so about DEPTH steps stay in flight (the
+  // barriers keep the scheduler from pairing each load with its use)
+  u32x4 w[DEPTH][NF], x[DEPTH][RB];
+  unsigned aofs[RB];
+  auto load_w = [&](int slot, int j) {
+    const unsigned k0w = (unsigned)(wave + WAVES * j) * 1024u;  // four k groups of 16 pieces
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      w[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(wr, j < mine ? wofs[f] + k0w : kOutside, 0, 2);
+  };
+  auto load_x = [&](int slot, int j) {
+    const unsigned k0b = (unsigned)(wave + WAVES * j) * 64u;  // bytes along an A row
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      x[slot][b] = __builtin_amdgcn_raw_buffer_load_b128(ar, j < mine ? aofs[b] + k0b : kOutside, 0, 0);
+  };
+  auto multiply = [&](int slot) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        acc[b][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[slot][b]),
+                                                            __builtin_bit_cast(bf16x8, w[slot][f]), acc[b][f], 0, 0, 0);
+  };
+#pragma unroll
+  for (int i = 0; i < DEPTH; ++i) load_w(i, i);
+  __builtin_amdgcn_sched_barrier(0);
+  // (after the weight loads: the rows' numbers are waited for here)
+#pragma unroll
+  for (int b = 0; b < RB; ++b) aofs[b] = 16 * b + fr < g.rows ? (row[b] * (unsigned)K + fk) * 2u : kOutside;
+#pragma unroll
+  for (int i = 0; i < DEPTH; ++i) load_x(i, i);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int j0 = 0; j0 + DEPTH < mine; j0 += DEPTH) {
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) {
+      multiply(i);
+      load_w(i, j0 + DEPTH + i);
+      load_x(i, j0 + DEPTH + i);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  red[0][wave][lane] = acc;
-  if constexpr (U) red[1][wave][lane] = accu;
+#pragma unroll
+  for (int i = 0; i < DEPTH; ++i) multiply(i);  // (slots past the last step hold zeros)
+  auto part = [&](int wv, int b, int f) -> f32x4& { return red[((wv * RB + b) * NF + f) * 64 + lane]; };
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) part(wave, b, f) = acc[b][f];
   __syncthreads();
-  if (wave != 0) return;
-  // D layout: lane holds rows 4 (lane / 16) + r, output lane % 16
-  f32x4 g = red[0][0][lane], up = U ? red[1][0][lane] : f32x4{0.f, 0.f, 0.f, 0.f};
+  // the waves add the (row block, output block) pairs over all waves, in wave
+  // order.  D layout: lane holds rows 4 (lane / 16) + r, output lane % 16
+  for (int it = wave; it < RB * NO; it += WAVES) {
+    const int b = it / NO, o = it % NO, n = n0 + 16 * o + fr;
+    f32x4 s0 = part(0, b, o), s1 = PAIR ? part(0, b, NO + o) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int w = 1; w < kSlabWavesE; ++w) {
-    g += red[0][w][lane];
-    if constexpr (U) up += red[1][w][lane];
-  }
-  const int n = n0 + fr;
+    for (int wv = 1; wv < WAVES; ++wv) {
+      s0 += part(wv, b, o);
+      if constexpr (PAIR) s1 += part(wv, b, NO + o);
+    }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = 4 * (lane >> 4) + r;
-    if (i >= count) continue;
-    uint16_t* y = a.Y + (size_t)(off + i) * a.ldy;
-    if constexpr (PAIR) {
-      if (n < N) y[n] = (uint16_t)f32_to_bf16(silu_mul(round_bf16(g[r]), round_bf16(up[r])));
-    } else {
-      if (n < N) y[n] = (uint16_t)f32_to_bf16(g[r]);
-      if (TWO && n + 16 < N) y[n + 16] = (uint16_t)f32_to_bf16(up[r]);
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * b + 4 * (lane >> 4) + r;
+      if (i >= g.rows || n >= N) continue;
+      const float y = PAIR ? silu_mul(round_bf16(s0[r]), round_bf16(s1[r])) : s0[r];
+      a.Y[(size_t)(g.offset + i) * N + n] = (uint16_t)f32_to_bf16(y);
     }
   }
 }
+
+// Expert GEMM over the plan's groups: workgroup (s, z) computes NF / 2 blocks
+// of 16 gate and up outputs (PAIR: SwiGLU bf16(silu(bf16(g)) * bf16(u))) or
+// NF blocks of plain ones of group z's expert, for the group's rows (at most
+// kGroupRows).  Wave w takes the 32-column K steps w, w + WAVES, ... and
+// multiplies on MFMA 16x16x32 (rows x outputs); the waves' partial sums meet
+// in LDS and are added in wave order.  A group runs on as many 16-row blocks
+// as it has rows for, with a shorter ring of steps in flight for more.
+//
+// HBM bounds it up to about 10 rows per expert: every expert's weights go by
+// once per group (66 experts of 2048 x 1408 in 120 us for gate/up, 6.3 TB/s).
+// With more rows the A fragments, re-read from L2 by every workgroup of the
+// group, weigh as much as the weights; WIDE halves them with twice the
+// outputs per workgroup, on half the waves with twice the registers (the same
+// two workgroups per CU).  Whole calls of a 2048 / 64 + 2 x 1408 / top-6
+// block, narrow and wide: 1 token 38.8 and 40.1 us, 24 169 and 170, 61 195
+// and 188, 100 210 and 199, 256 302 and 238 (750 on 64 x 64 tiles of the
+// row-major weights with the plan's slots by a serial walk).
+template <bool PAIR, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 256 : 512, WIDE ? 2 : 4) void expert_slab_kernel(ExpertGemmArgs a) {
+  constexpr int NF = WIDE ? 4 : 2, WAVES = WIDE ? 4 : 8;
+  __shared__ f32x4 red[WAVES * (kGroupRows / 16) * NF * 64];
+  const int4 e = reinterpret_cast<const int4*>(a.groups)[blockIdx.y];
+  const ExpertGroup g = {e.x, e.y, e.z, 0};
+  if (g.rows == 0) return;
+  const int n0 = blockIdx.x * 16 * (PAIR ? NF / 2 : NF);
+  if (g.rows <= 16)
+    expert_slab<PAIR, NF, WAVES, 1, 8>(a, g, n0, red);
+  else if (g.rows <= 32)
+    expert_slab<PAIR, NF, WAVES, 2, 6>(a, g, n0, red);
+  else
+    expert_slab<PAIR, NF, WAVES, 4, WIDE ? 4 : 3>(a, g, n0, red);
+}
+
+template <bool PAIR>
+int launch_expert_slab(const ExpertGemmArgs& a, int groups, bool wide, hipStream_t st) {
+  const int outs = (PAIR ? 16 : 32) * (wide ? 2 : 1);  // per workgroup
+  const dim3 grid((a.N + outs - 1) / outs, groups);
+  if (wide)
+    hipLaunchKernelGGL((expert_slab_kernel<PAIR, true>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((expert_slab_kernel<PAIR, false>), grid, dim3(512), 0, st, a);
+  MOE_CHECK(hipGetLastError());
+  return 0;
+}
+
+// Tokens from which the expert GEMMs run WIDE (expert_slab_kernel's figures:
+// even at 24 tokens, 4% of a call at 61).
+constexpr int kWideTokens = 33;
 
 }  // namespace
 }  // namespace hk
@@ -392,10 +470,7 @@ struct hk_moe {
   float* logits = nullptr;       // [max_tokens * experts] router outputs
   int32_t* ids = nullptr;        // [max_tokens * top_k]
   float* weights = nullptr;      // [max_tokens * top_k]
-  int32_t* grp_expert = nullptr;
-  int32_t* grp_count = nullptr;
-  int32_t* grp_offset = nullptr;
-  int32_t* n_groups = nullptr;
+  ExpertGroup* groups = nullptr;
   int32_t* a_rows = nullptr;     // [pairs]
   int32_t* pair_slot = nullptr;  // [max_tokens * (top_k + shared)]
   uint16_t* act = nullptr;       // [pairs, I]
@@ -405,81 +480,53 @@ struct hk_moe {
 namespace {
 
 void moe_free(hk_moe* m) {
-  void* bufs[] = {m->gate_up_n, m->down_n, m->logits, m->ids, m->weights, m->grp_expert, m->grp_count, m->grp_offset, m->n_groups,
-                  m->a_rows, m->pair_slot, m->act, m->out};
+  void* bufs[] = {m->gate_up_n, m->down_n, m->logits, m->ids, m->weights, m->groups, m->a_rows, m->pair_slot, m->act, m->out};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   delete m;
 }
 
-// The experts and the combine after the plan (hk_moe_forward plans in
-// topk_plan_kernel; `planned` false runs route_plan_kernel on `ids` first).
-// `max_rows`: the most rows any expert gets (at most T when every token
-// names an expert once).
-int moe_run(hk_moe* m, const uint16_t* x, int T, const int32_t* ids, const float* weights,
-            uint16_t* y, hipStream_t st, bool planned, int max_rows) {
+// Groups that T tokens can make: every run of kGroupRows rows of an expert.
+int max_groups(const hk_moe_desc& d, int T) {
+  const int pairs = T * d.top_k, runs = (T + kGroupRows - 1) / kGroupRows;
+  return std::min(d.experts, pairs) + pairs / kGroupRows + d.shared * runs;
+}
+
+// The expert GEMMs and the combine, after the plan.
+int moe_run(hk_moe* m, const uint16_t* x, int T, const float* weights, uint16_t* y, hipStream_t st) {
   const hk_moe_desc& d = m->d;
-  const int K = d.top_k, S = d.shared, E = d.experts;
-  if (!planned) {
-    hipLaunchKernelGGL(route_plan_kernel, dim3(1), dim3(kThreads), 0, st, ids, T, K, E, S, m->grp_expert,
-                       m->grp_count, m->grp_offset, m->n_groups, m->a_rows, m->pair_slot);
-    MOE_CHECK(hipGetLastError());
-  }
-  const int max_groups = std::min(E, T * K) + S;
-  PrefillGemmArgs gu = {};
+  const int groups = max_groups(d, T), slots = T * (d.top_k + d.shared);
+  ExpertGemmArgs gu = {};
   gu.A = x;
-  gu.lda = d.hidden;
-  gu.W = m->gate_up;
   gu.Wn = m->gate_up_n;
-  gu.w_stride = (long long)2 * d.intermediate * d.hidden;
   gu.Y = m->act;
-  gu.ldy = d.intermediate;
-  gu.M = T;
+  gu.groups = m->groups;
+  gu.a_rows = m->a_rows;
+  gu.w_stride = (long long)2 * d.intermediate * d.hidden;
   gu.N = d.intermediate;
   gu.K = d.hidden;
-  gu.epi = EPI_SWIGLU;
-  gu.a_rows = m->a_rows;
-  gu.grp_expert = m->grp_expert;
-  gu.grp_count = m->grp_count;
-  gu.grp_offset = m->grp_offset;
-  gu.n_groups = m->n_groups;
-  gu.max_groups = max_groups;
-  gu.max_rows = T;
-  // at most 16 rows per group: the expert slabs (every group's rows in one
-  // MFMA block); more: the grouped tile GEMM
-  const bool slab = max_rows <= kSlabMaxRowsE;  // (hidden and intermediate are multiples of 32)
-  if (slab) {
-    hipLaunchKernelGGL(expert_slab_kernel<true>, dim3((d.intermediate + 15) / 16, max_groups), dim3(kSlabThreads),
-                       0, st, gu);
-    MOE_CHECK(hipGetLastError());
-  } else {
-    PrefillGemmArgs g = gu;
-    g.Wn = nullptr;  // (the tile GEMM reads the row-major weights)
-    MOE_TRY(launch_prefill_gemm(g, st));
-  }
-  PrefillGemmArgs dn = gu;
+  gu.a_bytes = T * d.hidden * 2;
+  MOE_TRY(launch_expert_slab<true>(gu, groups, T >= kWideTokens, st));
+  ExpertGemmArgs dn = gu;
   dn.A = m->act;
-  dn.lda = d.intermediate;
-  dn.W = m->down;
   dn.Wn = m->down_n;
-  dn.w_stride = (long long)d.hidden * d.intermediate;
   dn.Y = m->out;
-  dn.ldy = d.hidden;
+  dn.a_rows = nullptr;
+  dn.w_stride = (long long)d.hidden * d.intermediate;
   dn.N = d.hidden;
   dn.K = d.intermediate;
-  dn.epi = EPI_BF16;
-  dn.a_rows = nullptr;
-  if (slab) {
-    hipLaunchKernelGGL((expert_slab_kernel<false, true>), dim3((d.hidden + 31) / 32, max_groups),
-                       dim3(kSlabThreads), 0, st, dn);
-    MOE_CHECK(hipGetLastError());
-  } else {
-    PrefillGemmArgs g = dn;
-    g.Wn = nullptr;
-    MOE_TRY(launch_prefill_gemm(g, st));
-  }
+  dn.a_bytes = slots * d.intermediate * 2;
+  MOE_TRY(launch_expert_slab<false>(dn, groups, T >= kWideTokens, st));
   hipLaunchKernelGGL(combine_kernel, dim3(T, (d.hidden + kThreads - 1) / kThreads), dim3(kThreads), 0, st, m->out,
-                     m->pair_slot, weights, d.hidden, K, S, y);
+                     m->pair_slot, weights, d.hidden, d.top_k, d.shared, y);
+  MOE_CHECK(hipGetLastError());
+  return 0;
+}
+
+int plan_route(hk_moe* m, const int32_t* ids, int T, hipStream_t st) {
+  const hk_moe_desc& d = m->d;
+  hipLaunchKernelGGL(route_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, ids, T, d.top_k, d.experts, d.shared,
+                     max_groups(d, T), m->groups, m->a_rows, m->pair_slot);
   MOE_CHECK(hipGetLastError());
   return 0;
 }
@@ -526,10 +573,7 @@ int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_
     MOE_TRY(moe_alloc(&m->logits, (size_t)d.max_tokens * d.experts));
     MOE_TRY(moe_alloc(&m->ids, (size_t)d.max_tokens * d.top_k));
     MOE_TRY(moe_alloc(&m->weights, (size_t)d.max_tokens * d.top_k));
-    MOE_TRY(moe_alloc(&m->grp_expert, groups));
-    MOE_TRY(moe_alloc(&m->grp_count, groups));
-    MOE_TRY(moe_alloc(&m->grp_offset, groups));
-    MOE_TRY(moe_alloc(&m->n_groups, 1));
+    MOE_TRY(moe_alloc(&m->groups, max_groups(d, d.max_tokens)));
     MOE_TRY(moe_alloc(&m->a_rows, pairs));
     MOE_TRY(moe_alloc(&m->pair_slot, pairs));
     MOE_TRY(moe_alloc(&m->act, pairs * d.intermediate));
@@ -555,11 +599,19 @@ int hk_moe_forward(hk_moe* m, const uint16_t* x, int32_t tokens, uint16_t* y, in
   hipLaunchKernelGGL(router_logits_kernel, dim3(tokens, (d.experts + kRouterRows - 1) / kRouterRows),
                      dim3(kThreads), 0, st, x, m->router, d.hidden, d.experts, m->logits);
   MOE_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(topk_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, m->logits, tokens, d.experts, d.top_k,
-                     d.shared, m->ids, m->weights, m->grp_expert, m->grp_count, m->grp_offset, m->n_groups,
-                     m->a_rows, m->pair_slot);
-  MOE_CHECK(hipGetLastError());
-  MOE_TRY(moe_run(m, x, tokens, m->ids, m->weights, y, st, true, tokens));  // (top-k ids are distinct)
+  // one token per wave of the plan's workgroup, or the top-k spread over the
+  // GPU and the plan after it (one launch more)
+  if (tokens <= kPlanTokens) {
+    hipLaunchKernelGGL(topk_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, m->logits, tokens, d.experts, d.top_k,
+                       d.shared, max_groups(d, tokens), m->ids, m->weights, m->groups, m->a_rows, m->pair_slot);
+    MOE_CHECK(hipGetLastError());
+  } else {
+    hipLaunchKernelGGL(topk_kernel, dim3((tokens + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0, st,
+                       m->logits, tokens, d.experts, d.top_k, m->ids, m->weights);
+    MOE_CHECK(hipGetLastError());
+    MOE_TRY(plan_route(m, m->ids, tokens, st));
+  }
+  MOE_TRY(moe_run(m, x, tokens, m->weights, y, st));
   const size_t nk = (size_t)tokens * d.top_k;
   if (ids_out)
     MOE_CHECK(hipMemcpyAsync(ids_out, m->ids, nk * sizeof(int32_t), hipMemcpyDeviceToDevice, st));
@@ -578,13 +630,10 @@ int hk_moe_experts(hk_moe* m, const uint16_t* x, int32_t tokens, const int32_t* 
   std::vector<int32_t> host(nk);
   MOE_CHECK(hipMemcpyAsync(host.data(), ids, nk * sizeof(int32_t), hipMemcpyDeviceToHost, st));
   MOE_CHECK(hipStreamSynchronize(st));
-  std::vector<int> rows(m->d.experts, 0);
-  int max_rows = tokens;  // the shared experts
-  for (int32_t e : host) {
+  for (int32_t e : host)
     if (e < 0 || e >= m->d.experts) return fail("hk_moe_experts: expert id out of range");
-    max_rows = std::max(max_rows, ++rows[e]);  // a token may name an expert twice
-  }
-  return moe_run(m, x, tokens, ids, weights, y, st, false, max_rows);
+  MOE_TRY(plan_route(m, ids, tokens, st));
+  return moe_run(m, x, tokens, weights, y, st);
 }
 
 void hk_moe_destroy(hk_moe* m) {

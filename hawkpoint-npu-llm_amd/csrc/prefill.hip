@@ -56,35 +56,20 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(PrefillGemmArgs a) {
   const int wm = (wave >> 1) * 32;  // wave's token offset in the tile
   const int wn = (wave & 1) * 32;   // wave's output offset in the tile
 
-  // Grouped mode: this workgroup's expert, row count and row offset.
-  const uint16_t* Wb = a.W;
-  int M = a.M;
-  int row_off = 0;
-  const bool grouped = a.grp_count != nullptr;
-  if (grouped) {
-    const int z = blockIdx.z;
-    if (z >= *a.n_groups) return;
-    M = a.grp_count[z];
-    if (m0 >= M) return;
-    row_off = a.grp_offset[z];
-    Wb = a.W + (size_t)a.grp_expert[z] * (size_t)a.w_stride;
-  }
-
+  const int M = a.M;
   // one 16-byte piece of each tile per thread: row = tid / 4, k8 = (tid % 4) * 8
   const int lr = tid >> 2;
   const int lk = (tid & 3) * 8;
   const bool a_ok = (m0 + lr) < M;
   const bool w_ok = (n0 + lr) < a.N;
-  int arow = a_ok ? m0 + lr : 0;
-  if (grouped) arow = a.a_rows ? a.a_rows[row_off + (a_ok ? m0 + lr : 0)] : row_off + arow;
-  const uint16_t* a_src = a.A + (size_t)arow * a.lda + lk;
+  const uint16_t* a_src = a.A + (size_t)(a_ok ? m0 + lr : 0) * a.lda + lk;
   const size_t w_off = (size_t)(w_ok ? n0 + lr : 0) * a.K + lk;
   const size_t u_off = (size_t)(w_ok ? n0 + lr + a.N : 0) * a.K + lk;
   auto wload = [&](size_t off) -> u32x4 {
     if constexpr (W8)
-      return load_stream_i8_bf16(reinterpret_cast<const int8_t*>(Wb) + off);
+      return load_stream_i8_bf16(reinterpret_cast<const int8_t*>(a.W) + off);
     else
-      return load_stream16(Wb + off);
+      return load_stream16(a.W + off);
   };
   const u32x4 zero = {0u, 0u, 0u, 0u};
 
@@ -135,10 +120,9 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(PrefillGemmArgs a) {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int mt = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
+        const int m = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
         const int n = n0 + wn + j * 16 + (lane & 15);
-        if (mt >= M || n >= a.N) continue;
-        const int m = row_off + mt;
+        if (m >= M || n >= a.N) continue;
         float v = acc[i][j][r], u = accu[i][j][r];
         if constexpr (W8) {
           v *= a.scale[n];
@@ -1644,30 +1628,23 @@ bool ring_gemm() {
 template <bool W8>
 int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
   const bool pair = a.epi == EPI_SWIGLU;
-  const bool slab_path = a.grp_count == nullptr && a.M <= kSlabMaxTokens;
+  const bool slab_path = a.M <= kSlabMaxTokens;
   if (a.kblock && !slab_path) return fail("prefill gemm: k-blocked operands need the slab path (M <= 64)");
-  if (a.rope.on && !slab_path && (a.grp_count != nullptr || !prefill_rope_fusable(a.M, a.K)))
+  if (a.rope.on && !slab_path && !prefill_rope_fusable(a.M, a.K))
     return fail("prefill gemm: RoPE needs the slab path (M <= 64) or 128-token tiles with K a multiple of 64");
   if (a.rope.on && (a.N != (a.rope.q_heads + 2 * a.rope.kv_heads) * kHeadDim || a.epi == EPI_SWIGLU))
     return fail("prefill gemm: RoPE needs the QKV projection");
-  if (a.slab_ws && (a.gamma || a.rope.on || pair || a.grp_count != nullptr || a.M > kSlabMaxTokens ||
+  if (a.slab_ws && (a.gamma || a.rope.on || pair || a.M > kSlabMaxTokens ||
                     a.slab_error == nullptr || a.slab_tag == 0))
     return fail("slab gemm: the K split is for plain slabs, with an error word and a nonzero tag");
-  if (a.grp_count == nullptr && a.M <= kSlabMaxTokens) {
+  if (slab_path) {
     if (a.gamma && a.K > kSlabNormMaxK) return fail("slab gemm: a normalised A operand needs K <= 1024");
     if (a.Wn && a.N % 16) return fail("slab gemm: the MFMA-native copy needs whole 16-row slabs");
     return pair ? launch_slab<true, W8>(a, stream) : launch_slab<false, W8>(a, stream);
   }
   if (a.gamma) return fail("prefill gemm: a normalised A operand needs the slab path (M <= 64)");
   dim3 grid((a.N + kTN - 1) / kTN, (a.M + kTM - 1) / kTM);
-  if (a.grp_count != nullptr) {
-    if (a.max_groups <= 0 || a.max_rows <= 0 || a.n_groups == nullptr || a.grp_expert == nullptr ||
-        a.grp_offset == nullptr)
-      return fail("grouped gemm: group description incomplete");
-    grid.y = (a.max_rows + kTM - 1) / kTM;
-    grid.z = a.max_groups;
-  }
-  if (a.grp_count == nullptr && a.split_ws != nullptr && !a.rope.on && a.K % kBK == 0 && split_parts(a.M, a.N, a.K) > 1 &&
+  if (a.split_ws != nullptr && !a.rope.on && a.K % kBK == 0 && split_parts(a.M, a.N, a.K) > 1 &&
       split_ws_need(a.M, a.N, a.K, pair) <= a.split_ws_floats) {
     // too few tiles to fill the GPU: K split over ~kSplitTarget workgroups
     const int parts = split_parts(a.M, a.N, a.K);
@@ -1689,7 +1666,7 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
     err = hipGetLastError();
     return err == hipSuccess ? 0 : hip_fail(err, "split reduce launch");
   }
-  if (!W8 && ring_gemm() && a.grp_count == nullptr && a.M >= kBM && a.K % kRK == 0) {
+  if (!W8 && ring_gemm() && a.M >= kBM && a.K % kRK == 0) {
     // the LDS-ring form of the 128-token tiles below (bf16 weights), with
     // the same choice of tile width
     const int mt = (a.M + kBM - 1) / kBM, slots = 2 * cu_count();
@@ -1718,7 +1695,7 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
       hipLaunchKernelGGL((gemm_ring_kernel<128, false, 5>), g, dim3(kThreads), 0, stream, a);
     else
       hipLaunchKernelGGL((gemm_ring_kernel<64, false, 6>), g, dim3(kThreads), 0, stream, a);
-  } else if (a.grp_count == nullptr && a.M >= kBM && a.K % kBK == 0) {
+  } else if (a.M >= kBM && a.K % kBK == 0) {
     // 128-token tiles, 64 or 128 outputs wide: two workgroups fit a CU, and
     // the wide tiles (about 1.7 times the work each) are taken when the
     // narrow ones would need at least twice as many rounds of workgroups
@@ -1750,7 +1727,6 @@ int launch_prefill_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0 || a.K <= 0) return fail("prefill gemm: sizes must be positive");
   if (a.K % kTK != 0) return fail("prefill gemm: K must be a multiple of 32");
   if (a.lda % 8 != 0) return fail("prefill gemm: lda must be a multiple of 8");
-  if (a.scale && a.grp_count) return fail("prefill gemm: int8 weights in grouped mode are not supported");
   return a.scale ? launch_gemm<true>(a, stream) : launch_gemm<false>(a, stream);
 }
 

@@ -56,12 +56,12 @@ def test_moe_block_matches_oracle(block, moe_weights, tokens):
 
 
 def test_moe_block_beyond_16_tokens_matches_oracle(moe_weights):
-    """24 tokens: groups of more than 16 rows run on the grouped tile GEMM
-    (up to 16 on the expert slabs), and the top-k waves take two tokens each."""
+    """24 tokens: groups of more than 16 rows (the shared experts), and the
+    top-k in a launch of its own."""
     from runtime.moe import MoEBlock
 
     router, gate_up, down = moe_weights
-    announce("moe block T=24 (grouped tile GEMM)")
+    announce("moe block T=24")
     b = MoEBlock(router, gate_up, down, top_k=6, shared=2, max_tokens=32)
     try:
         rng = np.random.default_rng(124)
@@ -95,9 +95,8 @@ def test_moe_experts_with_given_routing(block, moe_weights):
 
 def test_moe_experts_repeated_ids_beyond_16_rows(block, moe_weights):
     """Caller ids may name one expert several times per token: 3 tokens x 6
-    times expert 3 is 18 rows for one expert, more than the expert slabs
-    take, so the grouped tile GEMM runs; against the oracle's experts and
-    combine (oracle/moe.py moe_forward's order)."""
+    times expert 3 is 18 rows for one expert, more than one 16-row block;
+    against the oracle's experts and combine (oracle/moe.py moe_forward's order)."""
     from oracle.moe import expert_forward
 
     router, gate_up, down = moe_weights
@@ -116,6 +115,59 @@ def test_moe_experts_repeated_ids_beyond_16_rows(block, moe_weights):
         for s_ in range(2):
             acc = acc + expert_forward(gate_up[64 + s_], down[64 + s_], xt)
         assert rel_l2(bf16.from_bits(y[t]), bf16.from_bits(bf16.to_bits(acc))) <= 1e-2, t
+
+
+@pytest.mark.parametrize("tokens", [16, 17, 33, 65, 130, 256])
+@pytest.mark.parametrize("shape", [(96, 32, 5, 0, 3), (64, 160, 64, 2, 6)])
+def test_moe_row_groups_match_oracle(tokens, shape):
+    """Groups of 1..64 rows (each row-block count of the expert slabs) and
+    experts of more rows than one group, K of fewer and of more 32-column
+    steps than waves, with and without shared experts; then the same routing
+    given by the caller, with one token's experts all the same."""
+    from oracle.moe import expert_forward
+    from runtime.moe import MoEBlock, synthetic_moe
+
+    H, I, E, S, K = shape
+    announce(f"moe row groups T={tokens} {shape}")
+    router, gate_up, down = synthetic_moe(dict(hidden=H, intermediate=I, experts=E, shared=S), seed=3, std=0.1)
+    rng = np.random.default_rng(tokens)
+    x = bf16.to_bits(rng.normal(0, 1, (tokens, H)).astype(np.float32))
+    b = MoEBlock(router, gate_up, down, top_k=K, shared=S, max_tokens=256)
+    try:
+        y, ids, w = b.forward(x)
+        ids2 = ids.copy()
+        ids2[tokens // 2] = ids2[tokens // 2, 0]
+        y2 = b.experts(x, ids2, w)
+        y3 = b.experts(x, np.full_like(ids, ids[0, 0]), w) if tokens == 16 else None
+    finally:
+        b.close()
+    ref_y, ref_ids, ref_w = moe_forward(x, router, gate_up, down, top_k=K, shared=S)
+    for t in range(tokens):
+        if not np.array_equal(ids[t], ref_ids[t]):
+            _, _, probs = route(router, bf16.from_bits(x[t]), K)
+            assert min(_tie_gap(probs, k) for k in range(1, K + 1)) < 1e-6, (t, ids[t], ref_ids[t])
+            continue
+        np.testing.assert_allclose(w[t], ref_w[t], rtol=1e-5, atol=1e-7)
+        assert rel_l2(bf16.from_bits(y[t]), bf16.from_bits(ref_y[t])) <= 1e-2, t
+    same = [t for t in range(tokens) if t != tokens // 2]
+    np.testing.assert_array_equal(y2[same], y[same])
+
+    def all_on(e, t):
+        """Token t's output with every choice on expert e."""
+        xt = bf16.from_bits(x[t])
+        out = expert_forward(gate_up[e], down[e], xt)
+        acc = np.zeros(H, dtype=np.float32)
+        for k in range(K):
+            acc = acc + w[t, k] * out
+        for s in range(S):
+            acc = acc + expert_forward(gate_up[E + s], down[E + s], xt)
+        return bf16.from_bits(bf16.to_bits(acc))
+
+    t = tokens // 2
+    assert rel_l2(bf16.from_bits(y2[t]), all_on(ids2[t, 0], t)) <= 1e-2
+    if y3 is not None:  # more than one group of one expert (96 rows of the second shape)
+        for t in range(tokens):
+            assert rel_l2(bf16.from_bits(y3[t]), all_on(ids[0, 0], t)) <= 1e-2, t
 
 
 def test_w8_expert_gemv_reference_pattern(hk_lib):
