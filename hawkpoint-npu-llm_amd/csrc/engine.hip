@@ -397,8 +397,8 @@ size_t ptag_words(const hk_engine* e) {
 // clean, and report it.
 int check_persistent(hk_engine* e, const int32_t* result_host) {
   if (e->pshape < 0 || result_host[1] == 0) return 0;
-  // a split launch also leaves when a workgroup finds itself on another XCD
-  // than the split assumes: later steps run undivided
+  // a split launch also waits in vain where its workgroups do not cover the
+  // XCDs as the split assumes: later steps run undivided
   e->xcd_split = false;
   HK_CHECK(hipStreamSynchronize(e->stream));
   HK_CHECK(hipMemset(e->psync, 0, psync_words(e) * sizeof(unsigned int)));
@@ -1063,9 +1063,8 @@ int hk_engine_prefill(hk_engine* e, const int32_t* tokens_host, int32_t n, int32
   HK_CHECK(hipMemcpyAsync(result, e->result, sizeof(result), hipMemcpyDeviceToHost, e->stream));
   HK_CHECK(hipStreamSynchronize(e->stream));
   if (result[2] != 0) {
-    // a K-split slab waited too long for one of its parts, or found a part
-    // on another XCD: this prefill's KV slots and logits are invalid; later
-    // prefills run the slabs unsplit
+    // a K-split slab waited too long for one of its parts: this prefill's KV
+    // slots and logits are invalid; later prefills run the slabs unsplit
     e->slab_split = false;
     HK_CHECK(hipMemset(e->result + 2, 0, sizeof(int32_t)));
     HK_CHECK(hipDeviceSynchronize());

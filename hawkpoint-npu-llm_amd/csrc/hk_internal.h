@@ -236,13 +236,12 @@ struct PrefillGemmArgs {
   const void* Wn;
   // Long-K slab GEMM without RoPE, norm or SwiGLU only (the down
   // projection): with slab_ws, K is split kSlabParts ways over workgroups of
-  // one XCD (workgroup i runs on XCD i % 8).  Parts 1.. publish their float32
+  // one XCD.  Parts 1.. publish their float32
   // partial sums as tagged words (slab_tag << 32 | bits) into slab_ws, which
   // holds ceil(N / 16) * kSlabParts * kSlabMaxTokens * 16 of them; part 0
   // polls them from the XCD's L2, adds the parts in order and applies the
   // epilogue.  slab_tag is nonzero and new for every launch; a wait that
-  // gives up after slab_spin polls, or a workgroup found on another XCD,
-  // sets *slab_error.
+  // gives up after slab_spin polls sets *slab_error.
   unsigned long long* slab_ws;
   unsigned slab_tag, slab_spin;
   unsigned* slab_error;

@@ -65,6 +65,27 @@
 
 namespace hk {
 
+// MI355X: 8 XCDs of 32 CUs; the workgroups of a launch go round the XCDs in
+// turn, from a first XCD that depends on the hardware queue (a process's
+// first stream starts at XCD 0; with more queues in use each has a start of
+// its own).
+constexpr int kXcds = 8;
+// The workgroup's place in a step, on XCD place % 8: eight consecutive
+// workgroups run on eight XCDs whatever the first one is, so replacing the
+// low bits of the index by the XCD number renumbers them within their eight.
+// (Were two of the eight on one XCD, a place would stay empty and the waits
+// for it give up: the launch is abandoned.)  Not volatile, and its range
+// stated: the compiler may then read it again instead of keeping it (with a
+// volatile read the Qwen bf16 step spilled 192 scalars instead of 117 and
+// took 292 us instead of 286).
+__device__ __forceinline__ int xcd_place() {
+  unsigned xcc;
+  asm("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+  const unsigned place = (blockIdx.x & ~(kXcds - 1u)) | (xcc & (kXcds - 1u));
+  __builtin_assume(place < (unsigned)kPersistentGrid);
+  return (int)place;
+}
+
 // ---- phase stamps (built in only with -DHK_PHASE_STAMPS: lib/libhk_phases.so) ----
 // Thread 0 of each workgroup (or the thread named) writes the 100 MHz
 // real-time clock at fixed points of each of the first kStampLayers layers
@@ -87,12 +108,12 @@ __device__ unsigned long long hk_stamp_attn[kPersistentGrid][kStampLayers][kStam
 #define HK_STAMP_BY(tid, l, k)                                                                       \
   do {                                                                                               \
     if (threadIdx.x == (tid) && (l) < kStampLayers)                                                  \
-      hk_stamp_phase[blockIdx.x][l][k] = __builtin_amdgcn_s_memrealtime();                           \
+      hk_stamp_phase[xcd_place()][l][k] = __builtin_amdgcn_s_memrealtime();                          \
   } while (0)
 #define HK_STAMP_ATTN(l, k)                                                                          \
   do {                                                                                               \
     if (threadIdx.x == 0 && (l) < kStampLayers)                                                      \
-      hk_stamp_attn[blockIdx.x][l][k] = __builtin_amdgcn_s_memrealtime();                            \
+      hk_stamp_attn[xcd_place()][l][k] = __builtin_amdgcn_s_memrealtime();                           \
   } while (0)
 #else
 #define HK_STAMP_BY(tid, l, k) \
@@ -125,9 +146,6 @@ constexpr int kSc1 = 16;                  // buffer-load cache policy: device sc
 // with sc1 (written through to memory for other XCDs) is read with sc1 even
 // inside the XCD: an sc0|nt load can keep hitting a stale L2 copy of it.
 constexpr int kLocal = 3;
-// MI355X: 8 XCDs of 32 CUs; workgroup i of a one-per-CU launch runs on XCD
-// i % 8 (the XCD split checks this against the XCC_ID register).
-constexpr int kXcds = 8;
 constexpr int kXcdWg = kPersistentGrid / kXcds;
 static_assert(2 * kChunk == kPT, "two threads per attention slot");
 
@@ -1663,7 +1681,10 @@ __global__ __launch_bounds__(kPT) void decode_step_xa_kernel(PersistentArgs args
   Ctx c;
   c.a = &args;
   c.sm = &sm;
-  c.wg = blockIdx.x;
+  // With blockIdx.x as the place the split had to refuse every start but XCD
+  // 0: a process with several streams ran the undivided step, 426 us at
+  // position 71 of Qwen2.5-0.5B against 285.
+  c.wg = xcd_place();
   c.wave = threadIdx.x >> 6;
   c.lane = threadIdx.x & 63;
   const bool stager = c.wave >= kCW;
@@ -1687,15 +1708,6 @@ __global__ __launch_bounds__(kPT) void decode_step_xa_kernel(PersistentArgs args
     for (int i = threadIdx.x; i < L * kWords; i += kPT) dst[i] = ldg(src + i);
   }
   __syncthreads();
-  // the XCD-local hand-offs are only coherent if the workgroups that share
-  // them share an L2: leave (the launch is abandoned) if this workgroup is
-  // not on the XCD the split assumes
-  unsigned xcc;
-  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-  if ((xcc & 15u) != (unsigned)(c.wg % kXcds)) {
-    if (threadIdx.x == 0) give_up(a);
-    return;
-  }
   const uint16_t* x0 = token >= 0 ? a.embed + (size_t)min(token, a.vocab - 1) * S::H : a.h;
   const bool attn = c.wg % kXcds == 0;
   // rank of the workgroup within its side, and its compute waves' indices
@@ -2044,8 +2056,8 @@ __global__ void xcc_probe_kernel(unsigned* out) {
   if (threadIdx.x == 0) out[blockIdx.x] = xcc & 15u;
 }
 
-// 1 when workgroup i of a launch runs on XCD i % kXcds; else 0, with the
-// reason in hk_last_error().
+// 1 when each run of kXcds workgroups of a launch covers the XCDs once; else
+// 0, with the reason in hk_last_error().
 int xcd_layout_ok(hipStream_t stream) {
   unsigned* d = nullptr;
   if (hipMalloc(&d, kPersistentGrid * sizeof(unsigned)) != hipSuccess) {
@@ -2063,12 +2075,15 @@ int xcd_layout_ok(hipStream_t stream) {
     set_error(std::string("XCD split: layout probe failed: ") + hipGetErrorString(err));
     return 0;
   }
-  for (int i = 0; i < kPersistentGrid; ++i)
-    if (h[i] != (unsigned)(i % kXcds)) {
-      set_error("XCD split: workgroup " + std::to_string(i) + " ran on XCD " + std::to_string(h[i]) +
-                ", not " + std::to_string(i % kXcds));
+  for (int i = 0; i < kPersistentGrid; i += kXcds) {
+    unsigned seen = 0;
+    for (int j = 0; j < kXcds; ++j) seen |= 1u << h[i + j];
+    if (seen != (1u << kXcds) - 1u) {
+      set_error("XCD split: workgroups " + std::to_string(i) + ".. ran on XCD set " + std::to_string(seen) +
+                ", not one on each of " + std::to_string(kXcds));
       return 0;
     }
+  }
   return 1;
 }
 

@@ -887,19 +887,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_slab_kernel(PrefillGemmArgs a
   __shared__ float ssq[NORM ? kSlabWaves : 1][kSlabMaxTokens];
   __shared__ float inv_s[kSlabMaxTokens];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  // this workgroup's slab and K part: the KS parts of slab s are workgroups
-  // s % 8 + 8 (KS (s / 8) + q), q = 0..KS-1, all on XCD s % 8
+  // this workgroup's slab and K part: the KS parts of slab s are places
+  // s % 8 + 8 (KS (s / 8) + q), q = 0..KS-1, all on XCD s % 8: eight
+  // consecutive workgroups run on eight XCDs, from a start that depends on
+  // the hardware queue, and each takes the place of its eight that its XCD
+  // has (two on one XCD would leave a place empty: part 0's wait gives up)
   int slab = blockIdx.x, part = 0;
   if constexpr (KS > 1) {
-    const int xcd = blockIdx.x % 8, r = blockIdx.x / 8;
-    part = r % KS;
-    slab = xcd + 8 * (r / KS);
     unsigned xcc;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-    if ((xcc & 15u) != (unsigned)xcd) {  // the parts would not share an L2: report, leave
-      if (tid == 0) __hip_atomic_store(a.slab_error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
-    }
+    const int r = blockIdx.x / 8;
+    part = r % KS;
+    slab = (int)(xcc & 7u) + 8 * (r / KS);
     if (slab * 16 >= a.N) return;
   }
   const int n0 = slab * 16;

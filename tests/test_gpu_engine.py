@@ -217,7 +217,7 @@ def test_long_context_split_kv():
 
 
 def test_xcd_split_is_selected_by_context():
-    """On MI355X (8 XCDs, workgroup i on XCD i % 8) the Qwen step runs split
+    """On MI355X (8 XCDs, workgroups dealt to them in turn) the Qwen step runs split
     by XCD: with the attention tasks of a layer (14 query heads x 256-slot
     chunks) on XCD 0 while there are at most 48 (below position 768), on the
     224 MLP workgroups while they fit those (below 4096), and as one
@@ -253,6 +253,44 @@ def test_xcd_split_is_selected_by_context():
     finally:
         del os.environ["HK_XCD_SPLIT"]
 
+
+
+def test_xcd_split_beside_other_streams(hk_lib):
+    """A launch's first XCD depends on the hardware queue of its stream: with
+    streams on every queue, engines of each still run the split steps (short
+    and long form, and the K-split prefill slabs) and agree with the first."""
+    import ctypes
+
+    from runtime import hip
+    from runtime.qwen_engine import QwenDecoderEngine
+
+    announce("split step on several hardware queues")
+    model = SyntheticModel(QWEN25_05B, seed=6, layers=2)
+    prompt = _prompt(151936, 40, 21)
+    streams, engines, x = [], [], hip.DeviceBuffer.from_array(np.zeros(64, np.uint16))
+    try:
+        for _ in range(6):
+            handle = ctypes.c_void_p()
+            hip.check(hk_lib.hk_stream_create(ctypes.byref(handle)), "stream")
+            streams.append(handle.value)
+            hip.check(hk_lib.hk_rmsnorm(x.ptr, x.ptr, 1e-6, x.ptr, 64, handle.value), "norm")
+            engines.append(QwenDecoderEngine(model, context_length=1024))
+        results = []
+        for e in engines:
+            tok, logits = e.prefill(prompt, 0)
+            tokens = [tok] + e.generate(tok, 40, 4)
+            long_tok, long_logits = e.step_token(7, 800)
+            assert [e.step_kind(40), e.step_kind(800)] == ["xcd_split", "xcd_split_long"]
+            results.append((tokens, logits, long_tok, long_logits))
+        for tokens, logits, long_tok, long_logits in results[1:]:
+            assert tokens == results[0][0] and long_tok == results[0][2]
+            np.testing.assert_array_equal(logits, results[0][1])
+            np.testing.assert_array_equal(long_logits, results[0][3])
+    finally:
+        for e in engines:
+            e.close()
+        for s in streams:
+            hk_lib.hk_stream_destroy(s)
 
 
 def test_undivided_step_short_context(monkeypatch):
