@@ -59,8 +59,6 @@ __global__ void set_ctrl_kernel(StepCtrl* ctrl, int32_t token, int32_t position,
   ctrl->advance = advance;
 }
 
-__global__ void store_i32_kernel(int32_t* dst, int32_t value) { *dst = value; }
-
 // Zero n 32-bit words (a kernel rather than hipMemsetAsync, so that a
 // captured step graph can hold it).
 __global__ void clear_words_kernel(uint32_t* p, int n) {
@@ -76,7 +74,6 @@ __global__ void skip_epochs_kernel(unsigned int* progress, int n, int stride, un
 struct OpScratch {
   int device = -1;
   unsigned long long* keys = nullptr;
-  int32_t* position = nullptr;
   float* partial = nullptr;
   unsigned int* counters = nullptr;
   size_t partial_floats = 0;
@@ -92,7 +89,6 @@ int op_scratch(OpScratch** out, size_t partial_floats, int counter_slots) {
   OpScratch& s = g_op_scratch[dev];
   if (s.keys == nullptr) {
     HK_CHECK(hipMalloc(&s.keys, kMaxPartialKeys * sizeof(unsigned long long)));
-    HK_CHECK(hipMalloc(&s.position, sizeof(int32_t)));
   }
   if (partial_floats > s.partial_floats) {
     if (s.partial) HK_CHECK(hipFree(s.partial));
@@ -727,13 +723,11 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
 }
 
 // ---- static scratch of hk_attention_decode_noalloc ----
-// Layout: [0, 256) the position word; [256, 256 + 4 kScratchTickets) the
-// per-head split-KV tickets; then the split-KV partials, [q_heads][splits][66]
-// floats.  Every GPU holds its own copy until the process ends; calls on one
-// GPU share it.
-constexpr size_t kScratchTicketsOffset = 256;
+// Layout: the per-head split-KV tickets, then the split-KV partials,
+// [q_heads][splits][66] floats.  Every GPU holds its own copy until the
+// process ends; calls on one GPU share it.
 constexpr int kScratchTickets = 1024;
-constexpr size_t kScratchPartialOffset = kScratchTicketsOffset + 4 * kScratchTickets;
+constexpr size_t kScratchPartialOffset = 4 * kScratchTickets;
 constexpr size_t kScratchPartialBytes = size_t(1) << 20;
 constexpr size_t kScratchBytes = kScratchPartialOffset + kScratchPartialBytes;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -757,12 +751,6 @@ int scratch_address(void** out) {
   }
   *out = g_scratch_address[dev];
   return 0;
-}
-
-// Position word and cleared tickets for one attention call.
-__global__ void attention_scratch_kernel(int32_t* position_word, int32_t position, unsigned int* tickets, int n) {
-  if (threadIdx.x == 0) *position_word = position;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) tickets[i] = 0u;
 }
 
 // Argument checks shared by both attention entry points.
@@ -1353,15 +1341,13 @@ int hk_attention_decode(const uint16_t* qkv, const float* rope_cos, const float*
   const int splits = attention_splits(max_context);
   OpScratch* s = nullptr;
   HK_TRY(op_scratch(&s, (size_t)q_heads * splits * (kHeadDim + 2), q_heads));
-  hipLaunchKernelGGL(store_i32_kernel, dim3(1), dim3(1), 0, st, s->position, position);
-  HK_CHECK(hipGetLastError());
   AttnArgs a = {};
   a.qkv = qkv;
   a.cos_tab = rope_cos;
   a.sin_tab = rope_sin;
   a.kcache = kcache;
   a.vcache = vcache;
-  a.position = s->position;
+  a.pos = position;
   a.out = out;
   a.partial = s->partial;
   a.counters = s->counters;
@@ -1386,11 +1372,9 @@ int hk_attention_decode_noalloc(const uint16_t* qkv, const float* rope_cos, cons
   void* base = nullptr;
   HK_TRY(scratch_address(&base));
   unsigned char* b = static_cast<unsigned char*>(base);
-  int32_t* position_word = reinterpret_cast<int32_t*>(b);
-  unsigned int* tickets = reinterpret_cast<unsigned int*>(b + kScratchTicketsOffset);
+  unsigned int* tickets = reinterpret_cast<unsigned int*>(b);
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(attention_scratch_kernel, dim3(1), dim3(256), 0, st, position_word, position, tickets,
-                     (int)q_heads);
+  hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, st, tickets, (int)q_heads);
   HK_CHECK(hipGetLastError());
   AttnArgs a = {};
   a.qkv = qkv;
@@ -1398,7 +1382,7 @@ int hk_attention_decode_noalloc(const uint16_t* qkv, const float* rope_cos, cons
   a.sin_tab = rope_sin;
   a.kcache = kcache;
   a.vcache = vcache;
-  a.position = position_word;
+  a.pos = position;
   a.out = out;
   a.partial = reinterpret_cast<float*>(b + kScratchPartialOffset);
   a.counters = tickets;

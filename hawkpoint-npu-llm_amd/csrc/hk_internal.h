@@ -78,11 +78,13 @@ struct AttnArgs {
   const float* sin_tab;      // [max_ctx, 32]
   uint16_t* kcache;          // this layer: [Hkv, max_ctx, 64] bf16
   uint16_t* vcache;          // this layer: [Hkv, max_ctx, 64] bf16
-  const int32_t* position;   // device scalar
+  const int32_t* position;   // device scalar, or null: the position is `pos`
   uint16_t* out;             // [Hq * 64] bf16
   float* partial;            // [Hq, max_splits, 66] split-KV partials (contexts > 256)
   unsigned int* counters;    // [Hq] zero between launches
   int q_heads, kv_heads, max_ctx, max_splits;
+  int pos;
+  int splits;                // set by launch_attention_decode: chunks of the grid
 };
 
 constexpr int kHeadDim = 64;

@@ -251,9 +251,9 @@ int hk_attention_decode(const uint16_t* qkv, const float* rope_cos, const float*
 /* hk_attention_decode without any allocation, for callers that cannot call
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  Same arguments, results
- * and errors as hk_attention_decode; its scratch (the position word, one
- * split-KV ticket per query head and the split-KV partials) is a static
- * device array of 1 MiB + 4352 bytes per GPU, held until the process ends.
+ * and errors as hk_attention_decode; its scratch (one split-KV ticket
+ * per query head and the split-KV partials) is a static device array of
+ * 1 MiB + 4096 bytes per GPU, held until the process ends.
  * HK_ERR_INVALID when q_heads > 1024 or q_heads * ceil(max_context / 256) *
  * 264 bytes of partials exceed 1 MiB (Qwen2.5-0.5B's 14 heads: any context up
  * to 65536).  Calls on one GPU share the scratch: calls that overlap in time

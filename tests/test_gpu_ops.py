@@ -279,7 +279,10 @@ def _attention_case(hk_lib, q_heads, kv_heads, ctx, position, seed):
 @pytest.mark.parametrize(
     "q_heads,kv_heads,ctx,position",
     [(14, 2, 128, 0), (14, 2, 128, 70), (9, 3, 64, 50), (14, 2, 4096, 255), (14, 2, 4096, 256),
-     (14, 2, 4096, 1000), (14, 2, 4096, 4095), (16, 1, 512, 300)],
+     (14, 2, 4096, 1000), (14, 2, 4096, 4095), (16, 1, 512, 300),
+     # a wave's and a chunk's first and last slots, no cached slot at all; more
+     # chunks than a wave merges at once, and every thread's chunk taken
+     (4, 4, 64, 0), (9, 3, 320, 63), (9, 3, 320, 64), (3, 1, 2048, 511), (14, 2, 10240, 9001), (2, 1, 65536, 65535)],
 )
 def test_attention_decode_matches_oracle(hk_lib, q_heads, kv_heads, ctx, position):
     announce(f"attention Hq={q_heads} Hkv={kv_heads} ctx={ctx} p={position}")
