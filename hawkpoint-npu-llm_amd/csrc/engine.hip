@@ -602,7 +602,9 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
   HK_TRY(launch_embed_rows(tokens_dev, n, d.vocab, e->w.token_embedding, H, e->pf_x, s, fused_norm ? n : 0));
   for (int l = 0; l < d.layers; ++l) {
     const hk_layer_weights& lw = e->layers[l];
-    if (!fused_norm) HK_TRY(launch_rmsnorm_rows(e->pf_x, H, lw.input_norm, d.rms_eps, e->pf_xn, H, n, H, s));
+    // (the later layers' input norm follows the down projection before them)
+    if (!slab ? l == 0 : !fused_norm)
+      HK_TRY(launch_rmsnorm_rows(e->pf_x, H, lw.input_norm, d.rms_eps, e->pf_xn, H, n, H, s));
     PrefillGemmArgs q = {};
     q.A = fused_norm ? e->pf_x : e->pf_xn;
     q.gamma = fused_norm ? lw.input_norm : nullptr;
@@ -620,9 +622,9 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     q.epi = lw.qkv_bias ? EPI_BIAS : EPI_BF16;
     q.kblock = fused_norm ? 1 : 0;
     // RoPE and the KV append in the QKV epilogue (no q/k/v rows, no
-    // rope_append launch): the slab GEMMs with the fused norm, and the
-    // 128-token tiles
-    const bool rope_fused = fused_norm || prefill_rope_fusable(n, H);
+    // rope_append launch): the slab GEMMs with the fused norm, and the tiles
+    // of longer chunks
+    const bool rope_fused = fused_norm || (!slab && prefill_rope_fusable(q));
     if (rope_fused) {
       q.rope.cos_tab = e->w.rope_cos;
       q.rope.sin_tab = e->w.rope_sin;
@@ -671,10 +673,16 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     o.K = QD;
     o.epi = EPI_RESID;
     o.kblock = kb;
+    if (!slab) {
+      o.next_gamma = lw.post_attn_norm;
+      o.next_xn = e->pf_xn;
+      o.eps = d.rms_eps;
+    }
     o.split_ws = e->pf_split;
     o.split_ws_floats = e->pf_split_floats;
     HK_TRY(launch_prefill_gemm(o, s));
-    if (!fused_norm) HK_TRY(launch_rmsnorm_rows(e->pf_h1, H, lw.post_attn_norm, d.rms_eps, e->pf_xn, H, n, H, s));
+    if (slab && !fused_norm)
+      HK_TRY(launch_rmsnorm_rows(e->pf_h1, H, lw.post_attn_norm, d.rms_eps, e->pf_xn, H, n, H, s));
     PrefillGemmArgs g = {};
     g.A = fused_norm ? e->pf_h1 : e->pf_xn;
     g.gamma = fused_norm ? lw.post_attn_norm : nullptr;
@@ -708,6 +716,11 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     dn.K = I;
     dn.epi = EPI_RESID;
     dn.kblock = kb;
+    if (!slab && l + 1 < d.layers) {
+      dn.next_gamma = e->layers[l + 1].input_norm;
+      dn.next_xn = e->pf_xn;
+      dn.eps = d.rms_eps;
+    }
     dn.split_ws = e->pf_split;
     dn.split_ws_floats = e->pf_split_floats;
     if (slab && e->slab_split && e->slab_ws) {  // K split inside an XCD, a new tag per launch

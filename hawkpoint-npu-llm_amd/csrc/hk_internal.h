@@ -216,6 +216,10 @@ struct PrefillGemmArgs {
   // unsplit.
   float* split_ws;
   size_t split_ws_floats;
+  // EPI_RESID with more than 64 tokens: with next_gamma ([N]) the RMSNorm of
+  // the finished rows (eps below) also goes to next_xn ([M, N])
+  const uint16_t* next_gamma;
+  uint16_t* next_xn;
   // Prompts of at most kSlabMaxTokens tokens run on the slab GEMM (one
   // workgroup per 16 outputs over all of K; no workspace).  With `gamma` (K at
   // most kSlabNormMaxK) the A rows are RMSNorm inputs, normalised as they are
@@ -287,9 +291,9 @@ struct PrefillAttnArgs {
   int period;               // set by launch_prefill_attention: the CU count
 };
 
-// Whether a QKV GEMM of M > 64 tokens and K inputs can apply RoPE and the KV
-// append in its epilogue (PrefillGemmArgs::rope; the 128-token tiles).
-bool prefill_rope_fusable(int M, int K);
+// Whether a QKV GEMM of more than 64 tokens can apply RoPE and the KV append
+// in its epilogue (PrefillGemmArgs::rope).
+bool prefill_rope_fusable(const PrefillGemmArgs& a);
 // rope_append (unless rope_done) then causal attention for tokens start..start+n-1.
 int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream);
 int launch_embed_rows(const int32_t* tokens, int n, int vocab, const uint16_t* table, int H,

@@ -604,9 +604,8 @@ __device__ __forceinline__ void lds_ready(bf16x8& v) {
 #endif
 }
 
-template <int BN, bool PAIR, int NS, int RK = kRK>
+template <int BM, int BN, bool PAIR, int NS, int RK, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring_kernel(PrefillGemmArgs a) {
-  constexpr int BM = kBM;
   constexpr int WR = PAIR ? 2 * BN : BN;  // weight rows per tile
   constexpr int MB = BM / 64, NB = BN / 64;  // MFMA 32 x 32 blocks per wave (64 x BN / 2 outputs)
   constexpr int SA = BM * RK, SW = WR * RK;  // bf16 per stage
@@ -632,7 +631,13 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
   const int n0 = (grp * GN + in % gn) * BN;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   const int fr = lane & 31;
-  const int steps = a.K / RK;
+  // this part's stages (SPLIT: part blockIdx.y of gridDim.y)
+  int steps = a.K / RK, st0 = 0;
+  if constexpr (SPLIT) {
+    const int per_part = (steps + (int)gridDim.y - 1) / (int)gridDim.y;
+    st0 = (int)blockIdx.y * per_part;
+    steps = min(steps - st0, per_part);
+  }
 
   const __amdgpu_buffer_rsrc_t ra = rsrc(a.A, a.M * a.lda * 2);
   const __amdgpu_buffer_rsrc_t rw = rsrc(a.W, (PAIR ? 2 : 1) * a.N * a.K * 2);
@@ -643,13 +648,13 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
     const int r = RPL * (wave * AI + i) + lr;  // tile row
-    aoff[i] = (unsigned)(((m0 + r) * a.lda + 8 * (lp ^ ring_key<RK>(r))) * 2);
+    aoff[i] = (unsigned)(((m0 + r) * a.lda + st0 * RK + 8 * (lp ^ ring_key<RK>(r))) * 2);
   }
 #pragma unroll
   for (int i = 0; i < WI; ++i) {
     const int r = RPL * (wave * WI + i) + lr;  // tile row: gate rows first, then up rows
     const int row = PAIR ? (r < BN ? n0 + r : a.N + n0 + r - BN) : n0 + r;
-    woff[i] = (unsigned)((row * a.K + 8 * (lp ^ ring_key<RK>(r))) * 2);
+    woff[i] = (unsigned)((row * a.K + st0 * RK + 8 * (lp ^ ring_key<RK>(r))) * 2);
   }
   f32x16 acc[MB][NB], accu[PAIR ? MB : 1][PAIR ? NB : 1];
 #pragma unroll
@@ -725,6 +730,23 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
           if constexpr (PAIR)
             accu[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[h][i], uf[h][j], accu[i][j], 0, 0, 0);
         }
+  }
+  if constexpr (SPLIT) {
+    // lane holds rows 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), n = n0 + wn + 32 * j + fr;
+          if (m >= a.M || n >= a.N) continue;
+          const int outs = PAIR ? 2 * a.N : a.N;
+          float* part = a.split_ws + ((size_t)blockIdx.y * a.M + m) * outs;
+          part[n] = acc[i][j][r];
+          if constexpr (PAIR) part[a.N + n] = accu[i][j][r];
+        }
+    return;
   }
   __syncthreads();  // the ring becomes the epilogue's tile
   tile_epilogue<BM, BN, PAIR, false, MB, NB, 32>(a, acc, accu, &ring[0][0], m0, n0, wm, wn, tid, lane);
@@ -1267,6 +1289,65 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(PrefillGemmArgs 
   }
 }
 
+// The end of a K-split GEMM with a residual on the ring: row m of Y is
+// bf16(bf16(sum of the parts in part order) + resid), and with next_gamma its
+// RMSNorm goes to next_xn in the same pass (the next GEMM's input; one launch
+// and one pass over the rows less).  A workgroup of two waves per row; the
+// first chunks of a row (up to 2048 values) stay in registers between the
+// sum of squares and the norm.
+constexpr int kRowThreads = 128;
+__global__ __launch_bounds__(kRowThreads) void split_resid_norm_kernel(PrefillGemmArgs a, int parts) {
+  constexpr int kKeep = 2;
+  __shared__ float sums[kRowThreads / 64];
+  const int m = blockIdx.x, tid = threadIdx.x, chunks = a.N / 8;
+  uint16_t* y = a.Y + (size_t)m * a.ldy;
+  float ss = 0.0f;
+  u32x4 keep[kKeep];
+  auto finish = [&](int c) -> u32x4 {
+    float v[8] = {};
+    for (int s = 0; s < parts; ++s) {
+      const u32x4* p = reinterpret_cast<const u32x4*>(a.split_ws + ((size_t)s * a.M + m) * a.N + 8 * c);
+      const u32x4 lo = load16(p), hi = load16(p + 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += __uint_as_float(lo[e]);
+        v[4 + e] += __uint_as_float(hi[e]);
+      }
+    }
+    if (a.scale) {  // W8: the row scales, on the finished sums
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= a.scale[8 * c + e];
+    }
+    const u32x4 r = load16(a.resid + (size_t)m * a.ldr + 8 * c);
+    u32x4 o;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      o[w] = f32x2_to_bf16x2(round_bf16(v[2 * w]) + bf_lo(r[w]), round_bf16(v[2 * w + 1]) + bf_hi(r[w]));
+    *reinterpret_cast<u32x4*>(y + 8 * c) = o;
+    return o;
+  };
+#pragma unroll
+  for (int k = 0; k < kKeep; ++k) {
+    const int c = tid + k * kRowThreads;
+    keep[k] = c < chunks ? finish(c) : u32x4{0u, 0u, 0u, 0u};
+    ss += sq8(keep[k]);
+  }
+  for (int c = tid + kKeep * kRowThreads; c < chunks; c += kRowThreads) ss += sq8(finish(c));
+  if (!a.next_gamma) return;
+  ss = group_sum<64>(ss);
+  if ((tid & 63) == 0) sums[tid >> 6] = ss;
+  __syncthreads();
+  const float inv = 1.0f / sqrtf((sums[0] + sums[1]) / (float)a.N + a.eps);
+  uint16_t* o = a.next_xn + (size_t)m * a.N;
+#pragma unroll
+  for (int k = 0; k < kKeep; ++k) {
+    const int c = tid + k * kRowThreads;
+    if (c < chunks) *reinterpret_cast<u32x4*>(o + 8 * c) = norm8(keep[k], inv, load16(a.next_gamma + 8 * c));
+  }
+  for (int c = tid + kKeep * kRowThreads; c < chunks; c += kRowThreads)  // (its own stores read back)
+    *reinterpret_cast<u32x4*>(o + 8 * c) = norm8(load16(y + 8 * c), inv, load16(a.next_gamma + 8 * c));
+}
+
 // Token rows per tile: 64 for prompts that fit one such tile, else kBM.
 int split_bm(int M) { return M <= 64 ? 64 : kBM; }
 
@@ -1556,9 +1637,30 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
 
 }  // namespace
 
+namespace {
+int tiles_of(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+
+// K parts of a residual GEMM on the ring's 64 x 64 tiles (1: no split): a
+// long K with too few tiles to fill the GPU is split over about one workgroup
+// per CU for the fewest tiles (their partial sums cost a pass each), two per
+// CU beyond, every part at least twelve 64-deep stages.  down_proj (K 4864,
+// N 896), us with the parts taken and unsplit or with one part fewer: 65
+// tokens 10.6 (6), 256 12.2 (4) and 13.4 (3), 417 15.0 (4) and 16.0 (3), 1021
+// 22.6 (2) and 23.2 (1).
+int ring_parts(int M, int N, int K) {
+  const int t = tiles_of(M, N, 64, 64), stages = K / 64;
+  if (t > 448 || N % 8 != 0) return 1;
+  const int want = std::max(1, std::min({6, (t <= 64 ? 256 : 448) / t, stages / 12}));
+  const int per = (stages + want - 1) / std::max(want, 1);
+  return per > 0 ? (stages + per - 1) / per : 1;
+}
+}  // namespace
+
 size_t split_ws_need(int M, int N, int K, bool pair) {
   const int parts = split_parts(M, N, K);
-  return parts > 1 ? (size_t)parts * M * (pair ? 2 * N : N) : 0;
+  const size_t big = parts > 1 ? (size_t)parts * M * (pair ? 2 * N : N) : 0;
+  const int ring = pair ? 1 : ring_parts(M, N, K);
+  return std::max(big, ring > 1 ? (size_t)ring * M * N : 0);
 }
 
 namespace {
@@ -1624,13 +1726,89 @@ bool ring_gemm() {
   return on;
 }
 
+// Whether the ring takes a GEMM of more than 64 tokens: bf16 weights, operands
+// whose bytes fit a buffer resource, and 16-byte rows for its buffer -> LDS
+// loads.
+bool ring_takes(const PrefillGemmArgs& a) {
+  const bool fits = (long long)a.M * a.lda * 2 < (1ll << 31) &&
+                    (a.epi == EPI_SWIGLU ? 2ll : 1ll) * a.N * a.K * 2 < (1ll << 31);
+  return !a.scale && ring_gemm() && a.M > kSlabMaxTokens && a.K % kRK == 0 && fits &&
+         ((reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W)) & 15u) == 0;
+}
+
+template <int BM, int BN, bool PAIR, int NS, int RK>
+void launch_ring_tiles(const PrefillGemmArgs& a, hipStream_t stream) {
+  const dim3 g(8 * ((tiles_of(a.M, a.N, BM, BN) + 7) / 8));
+  hipLaunchKernelGGL((gemm_ring_kernel<BM, BN, PAIR, NS, RK>), g, dim3(kThreads), 0, stream, a);
+}
+
+// The ring's tiles.  Few tiles leave CUs idle and a workgroup alone with its
+// latencies, so the smallest ones are taken while they run at once, two per
+// CU; stages are 64 deep where K allows it (half the barriers per product).
+// us for 896 -> 1152 (QKV), 896 -> 896 (O), 896 -> 2 x 4864 (gate/up), 4864 ->
+// 896 (down, unsplit), 64 x 64 tiles against the larger ones that follow:
+//   65 tokens   6.5   6.7  10.6  -     128 x 64:   -     -   14.5   -
+//   417         6.7   6.8  21.9  16.4              9.2   9.5  19.6
+//   2048       10.9   8.7   -    30.9             10.6  10.5   -   34.8
+//   4064       17.0  15.9   -    62.7  64 x 128:  18.9  12.8   -   45.5
+// (before, on 128-token tiles with K split over a workspace pass: 12.0, 11.1,
+// 16.5 at 65 and 13.9, 13.3, 25.4 at 417.)
+int launch_ring(const PrefillGemmArgs& a, hipStream_t stream, bool* normed) {
+  const bool pair = a.epi == EPI_SWIGLU, deep = a.K % 64 == 0;
+  const int slots = 2 * cu_count(), t64 = tiles_of(a.M, a.N, 64, 64);
+  const int parts = a.epi == EPI_RESID && deep ? ring_parts(a.M, a.N, a.K) : 1;
+  if (parts > 1 && a.split_ws != nullptr && (size_t)parts * a.M * a.N <= a.split_ws_floats) {
+    hipLaunchKernelGGL((gemm_ring_kernel<64, 64, false, 3, 64, true>), dim3(8 * ((t64 + 7) / 8), parts), dim3(kThreads),
+                       0, stream, a);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return hip_fail(err, "split gemm launch");
+    *normed = true;
+    hipLaunchKernelGGL(split_resid_norm_kernel, dim3(a.M), dim3(kRowThreads), 0, stream, a, parts);
+    err = hipGetLastError();
+    return err == hipSuccess ? 0 : hip_fail(err, "split reduce launch");
+  }
+  if (t64 <= slots) {
+    if (pair && deep)
+      launch_ring_tiles<64, 64, true, 3, 64>(a, stream);
+    else if (pair)
+      launch_ring_tiles<64, 64, true, 4, 32>(a, stream);
+    else if (deep)
+      launch_ring_tiles<64, 64, false, 3, 64>(a, stream);
+    else
+      launch_ring_tiles<64, 64, false, 4, 32>(a, stream);
+  } else if (pair) {
+    // gate/up in 128 x (64 + 64) tiles, three per CU, while they run at once
+    // (417 tokens 19.6 against 25.7 us in the larger ones, 1021 31.8 and
+    // 33.9); then 128 x (128 + 128) ones, each wave 64 tokens x 64 gate + 64
+    // up outputs at two waves per SIMD (1500 tokens 38.8 against 40.3, 4064
+    // 82.6 and 84.7)
+    if (tiles_of(a.M, a.N, 128, 64) <= 3 * cu_count())
+      launch_ring_tiles<128, 64, true, 3, 32>(a, stream);
+    else
+      launch_ring_tiles<128, 128, true, 3, 32>(a, stream);
+  } else if (deep && tiles_of(a.M, a.N, 64, 128) <= slots) {
+    launch_ring_tiles<64, 128, false, 3, 64>(a, stream);  // (4064 tokens, 128 x 64 tiles: O 13.7, down 48.9 us)
+  } else {
+    // 128-wide tiles (about 1.7 times the work each) where the narrow ones
+    // would need at least twice as many rounds of two workgroups per CU
+    const int rounds64 = (tiles_of(a.M, a.N, 128, 64) + slots - 1) / slots;
+    const int rounds128 = (tiles_of(a.M, a.N, 128, 128) + slots - 1) / slots;
+    if (rounds64 >= 2 * rounds128)
+      launch_ring_tiles<128, 128, false, 5, 32>(a, stream);
+    else
+      launch_ring_tiles<128, 64, false, 6, 32>(a, stream);
+  }
+  const hipError_t err = hipGetLastError();
+  return err == hipSuccess ? 0 : hip_fail(err, "ring gemm launch");
+}
+
 template <bool W8>
-int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
+int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream, bool* normed) {
   const bool pair = a.epi == EPI_SWIGLU;
   const bool slab_path = a.M <= kSlabMaxTokens;
   if (a.kblock && !slab_path) return fail("prefill gemm: k-blocked operands need the slab path (M <= 64)");
-  if (a.rope.on && !slab_path && !prefill_rope_fusable(a.M, a.K))
-    return fail("prefill gemm: RoPE needs the slab path (M <= 64) or 128-token tiles with K a multiple of 64");
+  if (a.rope.on && !slab_path && !prefill_rope_fusable(a))
+    return fail("prefill gemm: RoPE needs the slab path (M <= 64), the ring or 128-token tiles with K a multiple of 64");
   if (a.rope.on && (a.N != (a.rope.q_heads + 2 * a.rope.kv_heads) * kHeadDim || a.epi == EPI_SWIGLU))
     return fail("prefill gemm: RoPE needs the QKV projection");
   if (a.slab_ws && (a.gamma || a.rope.on || pair || a.M > kSlabMaxTokens ||
@@ -1642,6 +1820,7 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
     return pair ? launch_slab<true, W8>(a, stream) : launch_slab<false, W8>(a, stream);
   }
   if (a.gamma) return fail("prefill gemm: a normalised A operand needs the slab path (M <= 64)");
+  if (!W8 && ring_takes(a)) return launch_ring(a, stream, normed);
   dim3 grid((a.N + kTN - 1) / kTN, (a.M + kTM - 1) / kTM);
   if (a.split_ws != nullptr && !a.rope.on && a.K % kBK == 0 && split_parts(a.M, a.N, a.K) > 1 &&
       split_ws_need(a.M, a.N, a.K, pair) <= a.split_ws_floats) {
@@ -1665,36 +1844,7 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
     err = hipGetLastError();
     return err == hipSuccess ? 0 : hip_fail(err, "split reduce launch");
   }
-  if (!W8 && ring_gemm() && a.M >= kBM && a.K % kRK == 0) {
-    // the LDS-ring form of the 128-token tiles below (bf16 weights), with
-    // the same choice of tile width
-    const int mt = (a.M + kBM - 1) / kBM, slots = 2 * cu_count();
-    const int rounds64 = (mt * ((a.N + 63) / 64) + slots - 1) / slots;
-    const int rounds128 = (mt * ((a.N + 127) / 128) + slots - 1) / slots;
-    // when the 128-wide tiles fit one per CU (N = hidden at 4096 tokens),
-    // 64-wide tiles on three 64-deep stages (72 KiB of LDS) run two per CU
-    // instead, with K a multiple of 64; else the 128-wide tiles take a
-    // deeper ring, 9 stages, 144 KiB of LDS
-    const bool one_per_cu = !pair && mt * ((a.N + 127) / 128) <= cu_count();
-    const bool deep64 = one_per_cu && a.K % 64 == 0;
-    const bool wide = !pair && !deep64 && (one_per_cu || rounds64 >= 2 * rounds128);
-    const int bn = wide ? 128 : 64;
-    // (SwiGLU: 128 gate and 128 up rows per tile, each wave 64 tokens x 64
-    // gate + 64 up outputs, three 24 KiB stages; the kernel is held to two
-    // waves per SIMD, i.e. two workgroups per CU)
-    const int bnt = pair ? 128 : bn;
-    const dim3 g(8 * ((mt * ((a.N + bnt - 1) / bnt) + 7) / 8));
-    if (pair)
-      hipLaunchKernelGGL((gemm_ring_kernel<128, true, 3>), g, dim3(kThreads), 0, stream, a);
-    else if (deep64)
-      hipLaunchKernelGGL((gemm_ring_kernel<64, false, 3, 64>), g, dim3(kThreads), 0, stream, a);
-    else if (one_per_cu)
-      hipLaunchKernelGGL((gemm_ring_kernel<128, false, 9>), g, dim3(kThreads), 0, stream, a);
-    else if (wide)
-      hipLaunchKernelGGL((gemm_ring_kernel<128, false, 5>), g, dim3(kThreads), 0, stream, a);
-    else
-      hipLaunchKernelGGL((gemm_ring_kernel<64, false, 6>), g, dim3(kThreads), 0, stream, a);
-  } else if (a.M >= kBM && a.K % kBK == 0) {
+  if (a.M >= kBM && a.K % kBK == 0) {
     // 128-token tiles, 64 or 128 outputs wide: two workgroups fit a CU, and
     // the wide tiles (about 1.7 times the work each) are taken when the
     // narrow ones would need at least twice as many rounds of workgroups
@@ -1720,13 +1870,19 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
 }
 }  // namespace
 
-bool prefill_rope_fusable(int M, int K) { return M > kSlabMaxTokens && M >= kBM && K % kBK == 0; }
+bool prefill_rope_fusable(const PrefillGemmArgs& a) { return ring_takes(a) || (a.M >= kBM && a.K % kBK == 0); }
 
 int launch_prefill_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0 || a.K <= 0) return fail("prefill gemm: sizes must be positive");
   if (a.K % kTK != 0) return fail("prefill gemm: K must be a multiple of 32");
   if (a.lda % 8 != 0) return fail("prefill gemm: lda must be a multiple of 8");
-  return a.scale ? launch_gemm<true>(a, stream) : launch_gemm<false>(a, stream);
+  if (a.next_gamma && (a.epi != EPI_RESID || a.M <= kSlabMaxTokens || !a.next_xn))
+    return fail("prefill gemm: the next RMSNorm needs a residual GEMM of more than 64 tokens");
+  bool normed = false;
+  if (const int rc = a.scale ? launch_gemm<true>(a, stream, &normed) : launch_gemm<false>(a, stream, &normed)) return rc;
+  if (a.next_gamma && !normed)
+    return launch_rmsnorm_rows(a.Y, a.ldy, a.next_gamma, a.eps, a.next_xn, a.N, a.M, a.N, stream);
+  return 0;
 }
 
 int launch_embed_rows(const int32_t* tokens, int n, int vocab, const uint16_t* table, int H,

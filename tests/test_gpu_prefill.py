@@ -30,7 +30,11 @@ def _dev(array):
      # several groups of output tiles: whole and ragged token tiles
      (2048, 1152, 896, "bias"), (1500, 2048, 192, "resid"),
      # 128-wide output tiles: 64-wide ones would take two rounds of workgroups
-     (4096, 1152, 128, "bias")],
+     (4096, 1152, 128, "bias"),
+     # 64-token tiles: one row past the slabs, rows and outputs off the tile and
+     # off the 16-byte pieces, stages of 32 columns, a single stage
+     (65, 64, 64, "resid"), (127, 999, 448, "none"), (70, 1001, 96, "resid"), (65, 130, 32, "bias"),
+     (2300, 899, 160, "bias")],
 )
 def test_gemm_bf16_matches_oracle(hk_lib, m, n, k, epi):
     from runtime import hip
@@ -139,6 +143,16 @@ def test_prefill_long_prompt():
     partly masked."""
     model = SyntheticModel(QWEN25_05B, seed=5, layers=2)
     _prefill_case(model, _prompt(151936, 600, 14), 4, 1024, 1e-2, "qwen-2L-600")
+
+
+@pytest.mark.parametrize("shape,n", [("qwen", 65), ("qwen", 130), ("qwen", 417), ("qwen", 1021), ("smollm", 200),
+                                     ("wide", 65), ("wide", 300)])
+def test_prefill_between_slabs_and_long_prompts(shape, n):
+    """65 to about a thousand tokens: the smaller tiles, the down projection
+    with K split into 6, 5, 4 and 2 parts (and 2 of SmolLM2's 1536 columns)
+    with the next layer's RMSNorm in its second pass."""
+    model = SyntheticModel({"qwen": QWEN25_05B, "smollm": SMOLLM2_135M, "wide": WIDE_1152}[shape], seed=9, layers=2)
+    _prefill_case(model, _prompt(model.metadata["vocab_size"], n, 60 + n), 4, 1100, 1e-2, f"{shape}-2L-{n}")
 
 
 def test_prefill_longer_than_one_chunk():
