@@ -136,6 +136,11 @@ int gemv_common(const void* W, const float* scale, const uint16_t* x, const floa
 
 using namespace hk;
 
+// A layer's projections as bf16 copies of the int8 ones.
+struct WideLayer {
+  const uint16_t *qkv, *o, *gate_up, *down;
+};
+
 struct hk_engine {
   std::mutex mu;
   hk_model_desc d{};
@@ -199,6 +204,10 @@ struct hk_engine {
   // per layer, MFMA-native copies of qkv (RoPE order), o, gate_up and down
   // for the slab GEMMs of chunks up to 64 tokens (empty: row-major weights)
   std::vector<std::array<void*, 4>> pf_native;
+  // W8: bf16 copies of the layer projections for the GEMMs of longer chunks
+  // (one allocation; null until the first such chunk)
+  uint16_t* pf_wide = nullptr;
+  std::vector<WideLayer> pf_wide_layers;
   // the down slab GEMM of short prompts with K split inside an XCD
   // (PrefillGemmArgs::slab_ws): on where the XCD split's placement check
   // passed, unless HK_SLAB_SPLIT=0; off for good after a wait gave up
@@ -469,7 +478,7 @@ void free_engine(hk_engine* e) {
                   e->counters, e->keys,    e->ctrl,     e->out_tokens, e->result,
                   e->pf_x,    e->pf_h1,    e->pf_xn,    e->pf_qkv,     e->pf_q,
                   e->pf_att,  e->pf_act,   e->pf_tokens, e->pf_split, e->players, e->psync, e->ptag,
-                  e->wpart,   e->xpart};
+                  e->wpart,   e->xpart, e->pf_wide};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (uint16_t* p : e->down_x)
@@ -520,10 +529,8 @@ int alloc_prefill_buffers(hk_engine* e, int rows) {
   const int QD = d.q_heads * kHeadDim;
   e->pf_split_floats = 1;
   for (int m = 1; m <= rows; ++m)
-    e->pf_split_floats = std::max({e->pf_split_floats, split_ws_need(m, e->qkv_rows, d.hidden, false),
-                                   split_ws_need(m, d.hidden, QD, false),
-                                   split_ws_need(m, d.intermediate, d.hidden, true),
-                                   split_ws_need(m, d.hidden, d.intermediate, false)});
+    e->pf_split_floats = std::max({e->pf_split_floats, split_ws_need(m, d.hidden, QD),
+                                   split_ws_need(m, d.hidden, d.intermediate)});
   HK_TRY(dalloc(&e->pf_split, e->pf_split_floats));
   // tagged partial sums of the K-split down slabs (N = hidden); tag 0 never
   // matches a launch's
@@ -587,6 +594,47 @@ int native_copies(hk_engine* e) {
   return 0;
 }
 
+// The bf16 copies of a W8 engine's layer projections that the GEMMs of chunks
+// over kSlabMaxTokens read, one allocation made the first time such a chunk
+// runs (QKV and O come from the XCD split's copies where the engine has
+// them).  Without the memory for it the chunk runs on the int8 weights and a
+// later one tries again.
+int wide_copies(hk_engine* e) {
+  const hk_model_desc& d = e->d;
+  if (!e->w8 || e->pf_wide != nullptr) return 0;
+  const bool have = !e->wide.empty();
+  const size_t nq = (size_t)e->qkv_rows * d.hidden, no = (size_t)d.hidden * d.q_heads * kHeadDim;
+  const size_t ng = (size_t)2 * d.intermediate * d.hidden, nd = (size_t)d.hidden * d.intermediate;
+  const size_t per = (have ? 0 : nq + no) + ng + nd;
+  if (hipMalloc(reinterpret_cast<void**>(&e->pf_wide), per * d.layers * sizeof(uint16_t)) != hipSuccess) {
+    (void)hipGetLastError();
+    e->pf_wide = nullptr;
+    return 0;
+  }
+  e->pf_wide_layers.resize(d.layers);
+  int rc = 0;
+  for (int l = 0; l < d.layers && rc == 0; ++l) {
+    const hk_layer_weights& lw = e->layers[l];
+    uint16_t* p = e->pf_wide + per * l;
+    auto widen = [&](const void* src, size_t n) -> const uint16_t* {
+      uint16_t* at = p;
+      if (rc == 0) rc = launch_widen_i8(src, at, n, e->stream);
+      p += n;
+      return at;
+    };
+    WideLayer& w = e->pf_wide_layers[l];
+    w.qkv = have ? e->wide[l] : widen(lw.qkv, nq);
+    w.o = have ? e->wide[l] + nq : widen(lw.o_proj, no);
+    w.gate_up = widen(lw.gate_up, ng);
+    w.down = widen(lw.down_proj, nd);
+  }
+  if (rc != 0) {
+    (void)hipFree(e->pf_wide);
+    e->pf_wide = nullptr;
+  }
+  return rc;
+}
+
 // All layers for tokens[0..n) (already on the device) at slots start..start+n-1.
 int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
   const hk_model_desc& d = e->d;
@@ -599,6 +647,7 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
   const bool fused_norm = n <= kSlabMaxTokens && H <= kSlabNormMaxK;
   const int kb = fused_norm ? 2 : 0;
   const bool slab = n <= kSlabMaxTokens, native = !e->pf_native.empty();
+  const WideLayer* wide = e->pf_wide ? e->pf_wide_layers.data() : nullptr;
   HK_TRY(launch_embed_rows(tokens_dev, n, d.vocab, e->w.token_embedding, H, e->pf_x, s, fused_norm ? n : 0));
   for (int l = 0; l < d.layers; ++l) {
     const hk_layer_weights& lw = e->layers[l];
@@ -613,6 +662,7 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     q.W = static_cast<const uint16_t*>(lw.qkv);
     q.Wn = fused_norm && native ? e->pf_native[l][0] : nullptr;
     q.scale = e->w8 ? lw.qkv_scale : nullptr;
+    q.Wx = wide ? wide[l].qkv : nullptr;
     q.bias = lw.qkv_bias;
     q.Y = e->pf_qkv;
     q.ldy = e->qkv_rows;
@@ -664,6 +714,7 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     o.W = static_cast<const uint16_t*>(lw.o_proj);
     o.Wn = slab && native ? e->pf_native[l][1] : nullptr;
     o.scale = e->w8 ? lw.o_scale : nullptr;
+    o.Wx = wide ? wide[l].o : nullptr;
     o.resid = e->pf_x;
     o.ldr = H;
     o.Y = e->pf_h1;
@@ -691,6 +742,7 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     g.W = static_cast<const uint16_t*>(lw.gate_up);
     g.Wn = slab && native ? e->pf_native[l][2] : nullptr;
     g.scale = e->w8 ? lw.gate_up_scale : nullptr;
+    g.Wx = wide ? wide[l].gate_up : nullptr;
     g.Y = e->pf_act;
     g.ldy = I;
     g.M = n;
@@ -707,6 +759,7 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     dn.W = static_cast<const uint16_t*>(lw.down_proj);
     dn.Wn = slab && native ? e->pf_native[l][3] : nullptr;
     dn.scale = e->w8 ? lw.down_scale : nullptr;
+    dn.Wx = wide ? wide[l].down : nullptr;
     dn.resid = e->pf_h1;
     dn.ldr = H;
     dn.Y = e->pf_x;
@@ -1040,7 +1093,7 @@ int hk_engine_prefill(hk_engine* e, const int32_t* tokens_host, int32_t n, int32
     HK_TRY(prefill_workspace(e));
     for (int c0 = 0; c0 < n; c0 += e->pf_rows) {
       const int m = std::min(e->pf_rows, n - c0);
-      if (m <= kSlabMaxTokens) HK_TRY(native_copies(e));
+      HK_TRY(m <= kSlabMaxTokens ? native_copies(e) : wide_copies(e));
       HK_CHECK(hipMemcpyAsync(e->pf_tokens, tokens_host + c0, m * sizeof(int32_t),
                               hipMemcpyHostToDevice, e->stream));
       HK_TRY(prefill_chunk(e, e->pf_tokens, m, start + c0));

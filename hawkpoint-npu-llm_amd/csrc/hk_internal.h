@@ -205,15 +205,15 @@ struct PrefillGemmArgs {
   // W8: W holds int8 [N, K] (SwiGLU [2N, K]) and scale the float32 scale of
   // each weight row, applied to the finished sum; null for bf16 weights
   const float* scale;
+  const uint16_t* Wx;     // W8, more than 64 tokens: the bf16 copy of W, or null
   const uint16_t* resid;  // [M, ldr] (EPI_RESID)
   uint16_t* Y;            // [M, ldy] bf16 output
   int M, N, K, lda, ldr, ldy;
   int epi;                // EPI_BF16, EPI_BIAS, EPI_RESID or EPI_SWIGLU
-  // Optional float32 workspace: when the GEMM has too few tiles to fill the
-  // GPU (short prompts, narrow outputs), K is split across workgroups that
-  // write partial sums here, and a second kernel adds them up in order and
-  // applies the epilogue.  Without it (or when it is too small) the GEMM runs
-  // unsplit.
+  // Optional float32 workspace: a long-K residual GEMM with too few tiles to
+  // fill the GPU splits K across workgroups that write partial sums here, and
+  // a second kernel adds them up in order and applies the epilogue.  Without
+  // it (or when it is too small) the GEMM runs unsplit.
   float* split_ws;
   size_t split_ws_floats;
   // EPI_RESID with more than 64 tokens: with next_gamma ([N]) the RMSNorm of
@@ -231,12 +231,11 @@ struct PrefillGemmArgs {
   // of an MFMA fragment are one 256-byte run (lda, ldy, ldr unused).  A only
   // with kblock = 1, all three with kblock = 2.
   int kblock;
-  // The QKV projection (slab GEMM, or 128-token tiles when
-  // prefill_rope_fusable): with rope.on the epilogue applies RoPE and writes
+  // The QKV projection (slab GEMM, or the ring when prefill_rope_fusable): with rope.on the epilogue applies RoPE and writes
   // the rotated queries to rope.qrot and the rotated keys and the values to
   // the caches at slots rope.start.. (rope_append_kernel's job; Y is not
   // written).  The slabs then take the rows of each RoPE pair together
-  // (rope_row); a 128-token tile holds whole heads.  N = (q_heads + 2
+  // (rope_row); a ring tile holds whole heads.  N = (q_heads + 2
   // kv_heads) * 64.
   // Slab GEMM only: the MFMA-native copy of W (launch_repack_mfma), or null
   const void* Wn;
@@ -267,11 +266,9 @@ constexpr int kSlabNormMaxK = 1024;
 // compute units of the current device
 int cu_count();
 
-constexpr int kSplitTarget = 256;  // workgroups the split aims for
-// float32 workspace the split-K path needs for an M x N GEMM (2N outputs
-// with SwiGLU) with K columns: one M x outputs slice per K part (0 when
-// the GEMM is not split).
-size_t split_ws_need(int M, int N, int K, bool pair);
+// float32 workspace the K-split path needs for an M x N residual GEMM with K
+// columns: one M x N slice per part (0 when the GEMM is not split).
+size_t split_ws_need(int M, int N, int K);
 
 int launch_prefill_gemm(const PrefillGemmArgs& a, hipStream_t stream);
 

@@ -12,10 +12,12 @@
 //                      start..start+n-1                                 :78-108
 //   attention_prefill  causal GQA: token i attends to slots 0..start+i    :110-129
 //
-// GEMM tiling (wave64, v_mfma_f32_16x16x32_bf16): a 256-thread workgroup owns
-// a 64-token x 64-output tile (two weight tiles for SwiGLU pairs); each wave
-// owns a 32x32 quarter as 2x2 MFMA blocks.  K advances 32 at a time through
-// LDS; A and W tiles arrive with one 16-byte load per thread each.
+// GEMMs: up to 64 tokens the slabs (gemm_slab_kernel), more the LDS ring
+// (gemm_ring_kernel).  gemm_kernel takes what the ring does not (operands of
+// 2 GiB and more, rows off 16 bytes, an int8 matrix without a bf16 copy): a
+// 256-thread workgroup owns a 64-token x 64-output tile (two weight tiles for
+// SwiGLU pairs), each wave a 32x32 quarter as 2x2 MFMA 16x16x32 blocks; K
+// advances 32 at a time through LDS.
 #include <algorithm>
 
 #include "hk_common.h"
@@ -242,27 +244,13 @@ __global__ __launch_bounds__(kThreads) void rope_append_kernel(PrefillAttnArgs a
   }
 }
 
-// Large-M GEMM (prompt chunks of 128+ tokens): a 256-thread workgroup owns
-// 128 tokens x BN outputs (for SwiGLU, BN gate and BN up rows); the waves
-// split it 2 x 2, so each owns 64 x BN/2 as 4 x BN/32 MFMA blocks (twice
-// that for SwiGLU).  K advances 64 at a time through two LDS buffers: the
-// next step's tiles are loaded into registers while this step's MFMAs run,
-// then written to the other buffer, so one barrier per step suffices.
-constexpr int kBM = 128;
-constexpr int kBK = 64;
-constexpr int kBRow = kBK + 8;  // bf16 per LDS row (rows 144 B apart: no bank conflicts)
-
-// The epilogue of the large-M GEMMs: the tile's outputs go through LDS (ep:
+// The epilogue of the ring GEMM: the tile's outputs go through LDS (ep:
 // BM x (BN + 8) bf16, free once every wave is past the last K step) so that
 // they leave as 16-byte stores of 8 outputs of a row, with the residual rows
 // read the same way.  Wave tiles: rows wm.., columns wn.. of the tile, MB x
-// NB MFMA 16 x 16 blocks (D layout: lane holds rows 4 (lane / 16) + r,
-// column lane % 16 of each block).
-// DM 32: the blocks are MFMA 32 x 32 ones (lane holds rows 8 (r / 4) +
-// 4 (lane / 32) + r % 4, column lane % 32, r = 0..15).
-template <int DM> struct DBlock { using T = f32x4; };
-template <> struct DBlock<32> { using T = f32x16; };
-
+// NB MFMA 32 x 32 blocks (D layout: lane holds rows 8 (r / 4) + 4 (lane / 32)
+// + r % 4, column lane % 32, r = 0..15).  With row scales (W8) they multiply
+// the finished sums.
 // The QKV epilogue with RoPE and the KV append (rope_append_kernel's
 // arithmetic) for outputs n .. n + 7 of token row m: src holds their
 // bf16(sum), partner the bf16(sum) of the RoPE partners n ^ 32 .. (the tiles
@@ -313,9 +301,9 @@ __device__ __forceinline__ void rope_chunk(const PrefillGemmArgs& a, const uint1
   *reinterpret_cast<u32x4*>(dst) = u32x4{o[0], o[1], o[2], o[3]};
 }
 
-template <int BM, int BN, bool PAIR, bool W8, int MB, int NB, int DM = 16>
-__device__ __forceinline__ void tile_epilogue(const PrefillGemmArgs& a, const typename DBlock<DM>::T (&acc)[MB][NB],
-                                              const typename DBlock<DM>::T (&accu)[PAIR ? MB : 1][PAIR ? NB : 1],
+template <int BM, int BN, bool PAIR, int MB, int NB>
+__device__ __forceinline__ void tile_epilogue(const PrefillGemmArgs& a, const f32x16 (&acc)[MB][NB],
+                                              const f32x16 (&accu)[PAIR ? MB : 1][PAIR ? NB : 1],
                                               uint16_t* ep, int m0, int n0, int wm, int wn, int tid, int lane) {
   // LDS holds, per output,
   // the bf16 that the epilogue's first rounding gives: the finished value
@@ -323,23 +311,23 @@ __device__ __forceinline__ void tile_epilogue(const PrefillGemmArgs& a, const ty
   // residual is added to) for EPI_BIAS and EPI_RESID.  The rounding points
   // are those of the other GEMM kernels.
   constexpr int ER = BN + 8;  // bf16 per LDS row of the tile
-  const int fr = lane & 15;
+  float sv[NB], su[PAIR ? NB : 1];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int n = min(n0 + wn + 32 * j + (lane & 31), a.N - 1);
+    sv[j] = a.scale ? a.scale[n] : 1.0f;
+    if constexpr (PAIR) su[j] = a.scale ? a.scale[a.N + n] : 1.0f;
+  }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int r = 0; r < (DM == 16 ? 4 : 16); ++r) {
-        const int ml = DM == 16 ? wm + 16 * i + (lane >> 4) * 4 + r : wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int nl = DM == 16 ? wn + 16 * j + fr : wn + 32 * j + (lane & 31);
-        const int n = min(n0 + nl, a.N - 1);
-        float v = acc[i][j][r];
+      for (int r = 0; r < 16; ++r) {
+        const int ml = wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), nl = wn + 32 * j + (lane & 31);
+        const float v = acc[i][j][r] * sv[j];
         float u = 0.0f;
-        if constexpr (PAIR) u = accu[i][j][r];
-        if constexpr (W8) {
-          v *= a.scale[n];
-          if constexpr (PAIR) u *= a.scale[a.N + n];
-        }
+        if constexpr (PAIR) u = accu[i][j][r] * su[j];
         uint32_t y;
         if constexpr (PAIR)
           y = a.epi == EPI_SWIGLU ? f32_to_bf16(silu_mul(round_bf16(v), round_bf16(u))) : f32_to_bf16(v);
@@ -396,158 +384,13 @@ __device__ __forceinline__ void tile_epilogue(const PrefillGemmArgs& a, const ty
   }
 }
 
-// SPLIT (too few tiles to fill the GPU): workgroup (x, y) takes tile x
-// (token tiles varying fastest) and the y-th of gridDim.y runs of K steps,
-// and stores float32 partial sums to split_ws[y][m][outputs] (SwiGLU: up
-// outputs at N + n) for split_reduce_kernel.
-template <int BM, int BN, bool PAIR, bool SPLIT, bool W8 = false>
-__global__ __launch_bounds__(kThreads) void gemm_big_kernel(PrefillGemmArgs a) {
-  constexpr int WR = PAIR ? 2 * BN : BN;  // weight rows per tile
-  constexpr int MB = BM / 32;             // 16-row blocks per wave
-  constexpr int NB = BN / 32;             // 16-wide output blocks per wave
-  constexpr int AL = BM * kBK / 8 / kThreads;  // 16-byte pieces per thread, A tile
-  constexpr int WL = WR * kBK / 8 / kThreads;  // and weight tile
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][BM][kBRow];
-  __shared__ __attribute__((aligned(16))) uint16_t Ws[2][WR][kBRow];
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int mt = (a.M + BM - 1) / BM, ntile = (a.N + BN - 1) / BN;
-  int m0, n0, kt0 = 0, kt1 = a.K / kBK;
-  if constexpr (SPLIT) {
-    m0 = (blockIdx.x % mt) * BM;
-    n0 = (blockIdx.x / mt) * BN;
-    const int per = (kt1 + gridDim.y - 1) / gridDim.y;
-    kt0 = blockIdx.y * per;
-    kt1 = min(kt1, kt0 + per);
-  } else {
-    // Workgroups go to the 8 XCDs in turn (workgroup b to XCD b % 8).  Tile
-    // order t = (b % 8) * per + b / 8 gives each XCD a contiguous run.  The
-    // order walks groups of up to 12 output tiles (4 when there are more)
-    // with the output tile fastest, so the tiles an XCD holds at once share a
-    // few token tiles and a few weight tiles, which its own L2 keeps.
-    const int per = (mt * ntile + 7) / 8;
-    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if (t >= mt * ntile) return;
-    const int GN = ntile <= 12 ? ntile : 4;
-    const int grp = t / (GN * mt), gn = min(GN, ntile - grp * GN), in = t - grp * GN * mt;
-    m0 = (in / gn) * BM;
-    n0 = (grp * GN + in % gn) * BN;
-  }
-  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-
-  // piece i of this thread: row tid / 8 + 32 i, k (tid % 8) * 8 of the tile
-  const int pr = tid >> 3, pk = (tid & 7) * 8;
-  const uint16_t* a_src[AL];
-  bool a_ok[AL];
-#pragma unroll
-  for (int i = 0; i < AL; ++i) {
-    const int m = m0 + pr + 32 * i;
-    a_ok[i] = m < a.M;
-    a_src[i] = a.A + (size_t)(a_ok[i] ? m : 0) * a.lda + pk;
-  }
-  const void* w_src[WL];  // bf16, or int8 (W8) at the same element offset
-  bool w_ok[WL];
-#pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int r = pr + 32 * i;  // tile row: gate rows first, then up rows
-    const int n = n0 + (PAIR ? r % BN : r);
-    w_ok[i] = n < a.N;
-    const size_t off = (size_t)((w_ok[i] ? n : 0) + (PAIR && r >= BN ? a.N : 0)) * a.K + pk;
-    if constexpr (W8)
-      w_src[i] = reinterpret_cast<const int8_t*>(a.W) + off;
-    else
-      w_src[i] = a.W + off;
-  }
-
-  u32x4 av[AL], wv[WL];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < AL; ++i) av[i] = a_ok[i] ? load16(a_src[i] + k0) : zero;
-#pragma unroll
-    for (int i = 0; i < WL; ++i) {
-      if constexpr (W8)
-        wv[i] = w_ok[i] ? load_stream_i8_bf16(static_cast<const int8_t*>(w_src[i]) + k0) : zero;
-      else
-        wv[i] = w_ok[i] ? load_stream16(static_cast<const uint16_t*>(w_src[i]) + k0) : zero;
-    }
-  };
-  auto store = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < AL; ++i) *reinterpret_cast<u32x4*>(&As[b][pr + 32 * i][pk]) = av[i];
-#pragma unroll
-    for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4*>(&Ws[b][pr + 32 * i][pk]) = wv[i];
-  };
-
-  f32x4 acc[MB][NB], accu[PAIR ? MB : 1][PAIR ? NB : 1];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (PAIR) accu[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-
-  if (kt0 < kt1) {  // always true: split_parts leaves no part empty
-    load(kt0 * kBK);
-    store(0);
-    __syncthreads();
-  }
-  for (int kt = kt0; kt < kt1; ++kt) {
-    const int b = (kt - kt0) & 1;
-    if (kt + 1 < kt1) load((kt + 1) * kBK);
-#pragma unroll
-    for (int ks = 0; ks < kBK; ks += 32) {
-      bf16x8 af[MB], bf[NB], uf[PAIR ? NB : 1];
-#pragma unroll
-      for (int i = 0; i < MB; ++i) af[i] = *reinterpret_cast<const bf16x8*>(&As[b][wm + 16 * i + fr][ks + fk]);
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        bf[j] = *reinterpret_cast<const bf16x8*>(&Ws[b][wn + 16 * j + fr][ks + fk]);
-        if constexpr (PAIR) uf[j] = *reinterpret_cast<const bf16x8*>(&Ws[b][BN + wn + 16 * j + fr][ks + fk]);
-      }
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-          if constexpr (PAIR)
-            accu[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], uf[j], accu[i][j], 0, 0, 0);
-        }
-    }
-    if (kt + 1 < kt1) store(b ^ 1);
-    __syncthreads();
-  }
-
-  // D layout: lane holds rows 4 (lane / 16) + r, column lane % 16 of each block
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = m0 + wm + 16 * i + (lane >> 4) * 4 + r;
-          const int n = n0 + wn + 16 * j + fr;
-          if (m >= a.M || n >= a.N) continue;
-          const int outs = PAIR ? 2 * a.N : a.N;
-          float* part = a.split_ws + ((size_t)blockIdx.y * a.M + m) * outs;
-          part[n] = acc[i][j][r];
-          if constexpr (PAIR) part[a.N + n] = accu[i][j][r];
-        }
-    return;
-  }
-  static_assert(BM * (BN + 8) <= 2 * BM * kBRow, "the tile fits the A buffers");
-  tile_epilogue<BM, BN, PAIR, W8, MB, NB>(a, acc, accu, &As[0][0][0], m0, n0, wm, wn, tid, lane);
-}
-
-// Large-M GEMM, bf16 weights, with a ring of NS LDS stages of RK (32 or 64)
-// K each filled by buffer -> LDS loads (16 bytes per lane, 1 KiB per
-// instruction): the workgroup keeps NS - 1 stages of loads in flight while
-// it multiplies one, where gemm_big_kernel's register staging keeps one.
-// Tiles, waves and epilogue as gemm_big_kernel (128 tokens x BN outputs,
-// 2 x 2 waves).  A stage row is RK bf16 = RK / 8 16-byte pieces; piece c of
+// GEMM of more than 64 tokens, bf16 weights (or an int8 matrix's bf16 copy),
+// with a ring of NS LDS stages of RK (32 or 64) K each filled by buffer -> LDS
+// loads (16 bytes per lane, 1 KiB per instruction): the workgroup keeps NS - 1
+// stages of loads in flight while it multiplies one.  A 256-thread workgroup
+// owns BM tokens x BN outputs (for SwiGLU, BN gate and BN up rows); its waves
+// split the tile 2 x 2.  SPLIT: part blockIdx.y of K, float32 partial sums to
+// split_ws[part][m][n].  A stage row is RK bf16 = RK / 8 16-byte pieces; piece c of
 // tile row r sits at position c ^ ring_key<RK>(r), so that a fragment read
 // (16 rows, one piece) touches distinct banks in every group of 8 lanes
 // (128 bytes) and of 16 lanes (256 bytes).  Every load goes through a buffer
@@ -555,8 +398,6 @@ __global__ __launch_bounds__(kThreads) void gemm_big_kernel(PrefillGemmArgs a) {
 // covers A rows RPL (w AI + i) .. and weight rows RPL (w WI + i) .. (RPL =
 // 512 / RK rows per load); each wave waits for its own loads of a stage, the
 // barrier after that for everyone's.
-constexpr int kRK = 32;  // K per ring stage of the SwiGLU pair and of the narrower tiles
-
 // The ring's piece position key of tile row r (only r % 16 matters).  32-deep
 // stages (four pieces per 64-byte row): 0 0 1 1 2 2 3 3 1 1 0 0 3 3 2 2, so
 // rows r and r + 2 (the same 128-byte bank window) get different keys, and
@@ -613,6 +454,7 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
   constexpr int AI = BM / RPL / (kThreads / 64), WI = WR / RPL / (kThreads / 64);
   constexpr int NH = RK / 16;  // 16-deep MFMA steps per stage
   constexpr int PER = AI + WI;  // loads per wave per stage
+  static_assert(!(SPLIT && PAIR), "K is split for plain tiles");
   static_assert(AI >= 1 && WI >= 1 && NS >= 3 && (NS - 2) * (AI + WI) < 64, "ring shape");
   static_assert(BM * (BN + 8) <= NS * (SA + SW), "the epilogue tile fits the ring");
   __shared__ __attribute__((aligned(16))) uint16_t ring[NS][SA + SW];
@@ -620,8 +462,12 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int mt = (a.M + BM - 1) / BM, ntile = (a.N + BN - 1) / BN;
-  // tile order as gemm_big_kernel (each XCD a contiguous run, grouped so the
-  // tiles an XCD holds at once share token and weight tiles)
+  // Workgroups go to the 8 XCDs in turn (workgroup b to XCD b % 8, up to a
+  // common start).  Tile order t = (b % 8) * per + b / 8 gives each XCD a
+  // contiguous run.  The order walks groups of up to 12 output tiles (4 when
+  // there are more) with the output tile fastest, so the tiles an XCD holds
+  // at once share a few token tiles and a few weight tiles, which its own L2
+  // keeps.
   const int per = (mt * ntile + 7) / 8;
   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
   if (t >= mt * ntile) return;
@@ -741,15 +587,12 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
         for (int r = 0; r < 16; ++r) {
           const int m = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), n = n0 + wn + 32 * j + fr;
           if (m >= a.M || n >= a.N) continue;
-          const int outs = PAIR ? 2 * a.N : a.N;
-          float* part = a.split_ws + ((size_t)blockIdx.y * a.M + m) * outs;
-          part[n] = acc[i][j][r];
-          if constexpr (PAIR) part[a.N + n] = accu[i][j][r];
+          a.split_ws[((size_t)blockIdx.y * a.M + m) * a.N + n] = acc[i][j][r];
         }
     return;
   }
   __syncthreads();  // the ring becomes the epilogue's tile
-  tile_epilogue<BM, BN, PAIR, false, MB, NB, 32>(a, acc, accu, &ring[0][0], m0, n0, wm, wn, tid, lane);
+  tile_epilogue<BM, BN, PAIR, MB, NB>(a, acc, accu, &ring[0][0], m0, n0, wm, wn, tid, lane);
 }
 
 // ---- slab GEMM: prompts of at most 64 tokens ----
@@ -1252,43 +1095,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_slab_kernel(PrefillGemmArgs a
   }
 }
 
-// Sum of the split-K partial sums of output (m, n) in slice order, then the
-// epilogue of the GEMM (the same rounding points as gemm_big_kernel's).
-__global__ __launch_bounds__(kThreads) void split_reduce_kernel(PrefillGemmArgs a, int parts) {
-  const int e = blockIdx.x * kThreads + threadIdx.x;
-  if (e >= a.M * a.N) return;
-  const int m = e / a.N, n = e % a.N;
-  const bool pair = a.epi == EPI_SWIGLU;
-  const int outs = pair ? 2 * a.N : a.N;
-  float v = 0.0f, u = 0.0f;
-  for (int s = 0; s < parts; ++s) {
-    const float* part = a.split_ws + ((size_t)s * a.M + m) * outs;
-    v += part[n];
-    if (pair) u += part[a.N + n];
-  }
-  if (a.scale) {  // W8: the row scales, on the finished sums
-    v *= a.scale[n];
-    if (pair) u *= a.scale[a.N + n];
-  }
-  uint16_t* y = a.Y + (size_t)m * a.ldy + n;
-  switch (a.epi) {
-    case EPI_BF16:
-      *y = (uint16_t)f32_to_bf16(v);
-      break;
-    case EPI_BIAS:
-      *y = (uint16_t)f32_to_bf16(round_bf16(v) + a.bias[n]);
-      break;
-    case EPI_RESID:
-      *y = (uint16_t)f32_to_bf16(round_bf16(v) + bf16_to_f32(a.resid[(size_t)m * a.ldr + n]));
-      break;
-    case EPI_SWIGLU:
-      *y = (uint16_t)f32_to_bf16(silu_mul(round_bf16(v), round_bf16(u)));
-      break;
-    default:
-      break;
-  }
-}
-
 // The end of a K-split GEMM with a residual on the ring: row m of Y is
 // bf16(bf16(sum of the parts in part order) + resid), and with next_gamma its
 // RMSNorm goes to next_xn in the same pass (the next GEMM's input; one launch
@@ -1346,22 +1152,6 @@ __global__ __launch_bounds__(kRowThreads) void split_resid_norm_kernel(PrefillGe
   }
   for (int c = tid + kKeep * kRowThreads; c < chunks; c += kRowThreads)  // (its own stores read back)
     *reinterpret_cast<u32x4*>(o + 8 * c) = norm8(load16(y + 8 * c), inv, load16(a.next_gamma + 8 * c));
-}
-
-// Token rows per tile: 64 for prompts that fit one such tile, else kBM.
-int split_bm(int M) { return M <= 64 ? 64 : kBM; }
-
-// Tiles of the un-split GEMM (64-wide outputs).
-int gemm_tiles(int M, int N) { return ((M + split_bm(M) - 1) / split_bm(M)) * ((N + 63) / 64); }
-
-// K parts of the split path: enough that the tiles times the parts reach
-// about kSplitTarget workgroups, every part holding ceil(nk / parts) steps
-// or, the last, fewer but at least one.  1 means no split.
-int split_parts(int M, int N, int K) {
-  const int tiles = gemm_tiles(M, N), nk = K / kBK;
-  const int want = std::max(1, std::min(nk, (kSplitTarget + tiles - 1) / tiles));
-  const int per = (nk + want - 1) / want;
-  return (nk + per - 1) / per;
 }
 
 // Causal GQA attention for a block of 64 query tokens (token i at slot
@@ -1656,11 +1446,9 @@ int ring_parts(int M, int N, int K) {
 }
 }  // namespace
 
-size_t split_ws_need(int M, int N, int K, bool pair) {
-  const int parts = split_parts(M, N, K);
-  const size_t big = parts > 1 ? (size_t)parts * M * (pair ? 2 * N : N) : 0;
-  const int ring = pair ? 1 : ring_parts(M, N, K);
-  return std::max(big, ring > 1 ? (size_t)ring * M * N : 0);
+size_t split_ws_need(int M, int N, int K) {
+  const int parts = ring_parts(M, N, K);
+  return parts > 1 ? (size_t)parts * M * N : 0;
 }
 
 namespace {
@@ -1716,8 +1504,8 @@ int launch_slab(const PrefillGemmArgs& a, hipStream_t stream) {
   return err == hipSuccess ? 0 : hip_fail(err, "slab gemm launch");
 }
 
-// HK_GEMM_RING=0 runs the long-prompt bf16 GEMMs on gemm_big_kernel
-// instead of gemm_ring_kernel (read once).
+// HK_GEMM_RING=0 runs the GEMMs of more than 64 tokens on gemm_kernel instead
+// of gemm_ring_kernel (read once).
 bool ring_gemm() {
   static const bool on = [] {
     const char* v = std::getenv("HK_GEMM_RING");
@@ -1726,14 +1514,15 @@ bool ring_gemm() {
   return on;
 }
 
-// Whether the ring takes a GEMM of more than 64 tokens: bf16 weights, operands
-// whose bytes fit a buffer resource, and 16-byte rows for its buffer -> LDS
-// loads.
+// Whether the ring takes a GEMM of more than 64 tokens: bf16 weights (W8: their
+// bf16 copy), operands whose bytes fit a buffer resource, and 16-byte rows for
+// its buffer -> LDS loads.
 bool ring_takes(const PrefillGemmArgs& a) {
   const bool fits = (long long)a.M * a.lda * 2 < (1ll << 31) &&
                     (a.epi == EPI_SWIGLU ? 2ll : 1ll) * a.N * a.K * 2 < (1ll << 31);
-  return !a.scale && ring_gemm() && a.M > kSlabMaxTokens && a.K % kRK == 0 && fits &&
-         ((reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W)) & 15u) == 0;
+  const uint16_t* w = a.scale ? a.Wx : a.W;
+  return w && ring_gemm() && a.M > kSlabMaxTokens && a.K % 32 == 0 && fits &&
+         ((reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;
 }
 
 template <int BM, int BN, bool PAIR, int NS, int RK>
@@ -1753,7 +1542,14 @@ void launch_ring_tiles(const PrefillGemmArgs& a, hipStream_t stream) {
 //   4064       17.0  15.9   -    62.7  64 x 128:  18.9  12.8   -   45.5
 // (before, on 128-token tiles with K split over a workspace pass: 12.0, 11.1,
 // 16.5 at 65 and 13.9, 13.3, 25.4 at 417.)
-int launch_ring(const PrefillGemmArgs& a, hipStream_t stream, bool* normed) {
+//
+// W8: the bf16 copy of the int8 weights (every int8 value is a bf16 exactly)
+// with the row scales in the epilogue, the products and rounding points of the
+// int8 kernels.  Widening each weight in every workgroup that loads it had
+// cost more than the matrix products: 1021 tokens, gate/up 88 us against 34.
+int launch_ring(const PrefillGemmArgs& args, hipStream_t stream, bool* normed) {
+  PrefillGemmArgs a = args;
+  if (a.scale) a.W = a.Wx;
   const bool pair = a.epi == EPI_SWIGLU, deep = a.K % 64 == 0;
   const int slots = 2 * cu_count(), t64 = tiles_of(a.M, a.N, 64, 64);
   const int parts = a.epi == EPI_RESID && deep ? ring_parts(a.M, a.N, a.K) : 1;
@@ -1808,7 +1604,7 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream, bool* normed) {
   const bool slab_path = a.M <= kSlabMaxTokens;
   if (a.kblock && !slab_path) return fail("prefill gemm: k-blocked operands need the slab path (M <= 64)");
   if (a.rope.on && !slab_path && !prefill_rope_fusable(a))
-    return fail("prefill gemm: RoPE needs the slab path (M <= 64), the ring or 128-token tiles with K a multiple of 64");
+    return fail("prefill gemm: RoPE needs the slab path (M <= 64) or the ring");
   if (a.rope.on && (a.N != (a.rope.q_heads + 2 * a.rope.kv_heads) * kHeadDim || a.epi == EPI_SWIGLU))
     return fail("prefill gemm: RoPE needs the QKV projection");
   if (a.slab_ws && (a.gamma || a.rope.on || pair || a.M > kSlabMaxTokens ||
@@ -1820,57 +1616,18 @@ int launch_gemm(const PrefillGemmArgs& a, hipStream_t stream, bool* normed) {
     return pair ? launch_slab<true, W8>(a, stream) : launch_slab<false, W8>(a, stream);
   }
   if (a.gamma) return fail("prefill gemm: a normalised A operand needs the slab path (M <= 64)");
-  if (!W8 && ring_takes(a)) return launch_ring(a, stream, normed);
-  dim3 grid((a.N + kTN - 1) / kTN, (a.M + kTM - 1) / kTM);
-  if (a.split_ws != nullptr && !a.rope.on && a.K % kBK == 0 && split_parts(a.M, a.N, a.K) > 1 &&
-      split_ws_need(a.M, a.N, a.K, pair) <= a.split_ws_floats) {
-    // too few tiles to fill the GPU: K split over ~kSplitTarget workgroups
-    const int parts = split_parts(a.M, a.N, a.K);
-    const dim3 g(gemm_tiles(a.M, a.N), parts);
-    if (split_bm(a.M) == 64) {
-      if (pair)
-        hipLaunchKernelGGL((gemm_big_kernel<64, 64, true, true, W8>), g, dim3(kThreads), 0, stream, a);
-      else
-        hipLaunchKernelGGL((gemm_big_kernel<64, 64, false, true, W8>), g, dim3(kThreads), 0, stream, a);
-    } else if (pair) {
-      hipLaunchKernelGGL((gemm_big_kernel<kBM, 64, true, true, W8>), g, dim3(kThreads), 0, stream, a);
-    } else {
-      hipLaunchKernelGGL((gemm_big_kernel<kBM, 64, false, true, W8>), g, dim3(kThreads), 0, stream, a);
-    }
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return hip_fail(err, "split gemm launch");
-    hipLaunchKernelGGL(split_reduce_kernel, dim3((a.M * a.N + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                       stream, a, parts);
-    err = hipGetLastError();
-    return err == hipSuccess ? 0 : hip_fail(err, "split reduce launch");
-  }
-  if (a.M >= kBM && a.K % kBK == 0) {
-    // 128-token tiles, 64 or 128 outputs wide: two workgroups fit a CU, and
-    // the wide tiles (about 1.7 times the work each) are taken when the
-    // narrow ones would need at least twice as many rounds of workgroups
-    const int mt = (a.M + kBM - 1) / kBM, slots = 2 * cu_count();
-    const int rounds64 = (mt * ((a.N + 63) / 64) + slots - 1) / slots;
-    const int rounds128 = (mt * ((a.N + 127) / 128) + slots - 1) / slots;
-    const bool wide = !pair && rounds64 >= 2 * rounds128;
-    const int bn = wide ? 128 : 64;
-    const dim3 g(8 * ((mt * ((a.N + bn - 1) / bn) + 7) / 8));
-    if (pair)
-      hipLaunchKernelGGL((gemm_big_kernel<kBM, 64, true, false, W8>), g, dim3(kThreads), 0, stream, a);
-    else if (wide)
-      hipLaunchKernelGGL((gemm_big_kernel<kBM, 128, false, false, W8>), g, dim3(kThreads), 0, stream, a);
-    else
-      hipLaunchKernelGGL((gemm_big_kernel<kBM, 64, false, false, W8>), g, dim3(kThreads), 0, stream, a);
-  } else if (pair) {
+  if (ring_takes(a)) return launch_ring(a, stream, normed);
+  const dim3 grid((a.N + kTN - 1) / kTN, (a.M + kTM - 1) / kTM);
+  if (pair)
     hipLaunchKernelGGL((gemm_kernel<true, W8>), grid, dim3(kThreads), 0, stream, a);
-  } else {
+  else
     hipLaunchKernelGGL((gemm_kernel<false, W8>), grid, dim3(kThreads), 0, stream, a);
-  }
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0 : hip_fail(err, "prefill gemm launch");
 }
 }  // namespace
 
-bool prefill_rope_fusable(const PrefillGemmArgs& a) { return ring_takes(a) || (a.M >= kBM && a.K % kBK == 0); }
+bool prefill_rope_fusable(const PrefillGemmArgs& a) { return ring_takes(a); }
 
 int launch_prefill_gemm(const PrefillGemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0 || a.K <= 0) return fail("prefill gemm: sizes must be positive");

@@ -155,6 +155,17 @@ def test_prefill_between_slabs_and_long_prompts(shape, n):
     _prefill_case(model, _prompt(model.metadata["vocab_size"], n, 60 + n), 4, 1100, 1e-2, f"{shape}-2L-{n}")
 
 
+@pytest.mark.parametrize("n,split", [(65, "1"), (417, "1"), (700, "0")])
+def test_prefill_w8_over_64_tokens(n, split, monkeypatch):
+    """W8 prompts over 64 tokens on bf16 copies of the int8 rows with the row
+    scales in the epilogue (and in the split down projection's second pass);
+    QKV and O from the XCD split's copies, and without the split from the
+    prefill's own."""
+    monkeypatch.setenv("HK_XCD_SPLIT", split)
+    model = SyntheticModel(QWEN25_05B, seed=10, layers=2)
+    _prefill_case(model, _prompt(151936, n, 70 + n), 4, 1100, 1e-2, f"qwen-2L-w8-{n}", w8=True)
+
+
 def test_prefill_longer_than_one_chunk():
     """4200 tokens in one call run as a 4096-token chunk and a 104-token chunk
     that attends to it; the same prompt over two calls (1000 + 3200, each a
