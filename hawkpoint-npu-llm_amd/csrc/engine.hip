@@ -13,6 +13,8 @@
 // position; the host only rewrites the control block between replays.
 #include <algorithm>
 #include <array>
+#include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -136,6 +138,8 @@ int gemv_common(const void* W, const float* scale, const uint16_t* x, const floa
 
 using namespace hk;
 
+constexpr int kOutHead = 64;  // words before the logits in the output block
+
 // A layer's projections as bf16 copies of the int8 ones.
 struct WideLayer {
   const uint16_t *qkv, *o, *gate_up, *down;
@@ -166,7 +170,17 @@ struct hk_engine {
   unsigned long long* keys = nullptr;  // [kMaxPartialKeys] LM-head argmax partials
   StepCtrl* ctrl = nullptr;
   int32_t* out_tokens = nullptr;  // [max_ctx]
-  int32_t* result = nullptr;      // [3]: last argmax token, persistent-step error word, prefill split error word
+  // What a call brings back, as one block so that it is one copy: the result
+  // words (at most kOutHead of them: last argmax token, persistent-step error
+  // word, prefill split error word), then the logits
+  float* out_block = nullptr;
+  int32_t* result = nullptr;
+  // pinned host memory that the calls' copies go through: the block's copy
+  // (or a generate's tokens after the result words), then the inputs of one
+  // call (prompt tokens or an embedding row)
+  char* stage = nullptr;
+  size_t stage_inputs = 0;   // offset of the inputs
+  bool stage_pinned = false;
   // whole step in one persistent launch (persistent.hip); -1: per-kernel graph
   int pshape = -1;
   // the step may also run split by XCD (attention block on XCD 0); it does so
@@ -474,8 +488,8 @@ void free_engine(hk_engine* e) {
     if (g) (void)hipGraphExecDestroy(g);
   for (auto& kv : e->repeat_graphs) (void)hipGraphExecDestroy(kv.second);
   void* bufs[] = {e->h,       e->h1,       e->qkv,      e->attn,       e->act,
-                  e->normed,  e->logits,   e->kcache,   e->vcache,     e->partial,
-                  e->counters, e->keys,    e->ctrl,     e->out_tokens, e->result,
+                  e->normed,  e->out_block, e->kcache,   e->vcache,     e->partial,
+                  e->counters, e->keys,    e->ctrl,     e->out_tokens,
                   e->pf_x,    e->pf_h1,    e->pf_xn,    e->pf_qkv,     e->pf_q,
                   e->pf_att,  e->pf_act,   e->pf_tokens, e->pf_split, e->players, e->psync, e->ptag,
                   e->wpart,   e->xpart, e->pf_wide};
@@ -488,6 +502,12 @@ void free_engine(hk_engine* e) {
   for (auto& m : e->pf_native)
     for (void* p : m)
       if (p) (void)hipFree(p);
+  if (e->stage) {
+    if (e->stage_pinned)
+      (void)hipHostFree(e->stage);
+    else
+      std::free(e->stage);
+  }
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }
@@ -495,6 +515,50 @@ void free_engine(hk_engine* e) {
 template <typename T>
 int dalloc(T** p, size_t count) {
   HK_CHECK(hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T)));
+  return 0;
+}
+
+// The staging memory of an engine.  Copies between the device and pageable
+// memory go through the runtime's own staging, a wait each: 45 us for the
+// logits of a 151936-token vocabulary and about 10 for the result words, of a
+// 385 us decode step; with pinned memory the block is one copy of 25 us and a
+// memcpy of 6.  Without pinned memory the copies work as they did.
+int host_stage(hk_engine* e) {
+  const size_t words = kOutHead + (size_t)std::max(e->d.vocab, e->d.max_context);
+  const size_t inputs = std::max((size_t)e->d.max_context * sizeof(int32_t), (size_t)e->d.hidden * sizeof(uint16_t));
+  e->stage_inputs = (words * sizeof(float) + 255) / 256 * 256;
+  e->stage_pinned = hipHostMalloc(reinterpret_cast<void**>(&e->stage), e->stage_inputs + inputs, hipHostMallocDefault) ==
+                    hipSuccess;
+  if (!e->stage_pinned) {
+    (void)hipGetLastError();
+    e->stage = static_cast<char*>(std::malloc(e->stage_inputs + inputs));
+    if (!e->stage) return fail("hk_engine_create: no host memory");
+  }
+  return 0;
+}
+
+// Waits for the stream and brings back the result words, and the logits or
+// `n_tokens` of out_tokens where the caller wants them.
+int fetch_outputs(hk_engine* e, int32_t (&result)[3], float* logits_host, int32_t* tokens_host = nullptr,
+                  int n_tokens = 0) {
+  char* body = e->stage + kOutHead * sizeof(float);
+  const size_t logits = logits_host ? (size_t)e->d.vocab * sizeof(float) : 0;
+  HK_CHECK(hipMemcpyAsync(e->stage, e->out_block, logits ? kOutHead * sizeof(float) + logits : sizeof(result),
+                          hipMemcpyDeviceToHost, e->stream));
+  if (tokens_host)
+    HK_CHECK(hipMemcpyAsync(body, e->out_tokens, n_tokens * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
+  HK_CHECK(hipStreamSynchronize(e->stream));
+  std::memcpy(result, e->stage, sizeof(result));
+  if (logits_host) std::memcpy(logits_host, body, logits);
+  if (tokens_host) std::memcpy(tokens_host, body, n_tokens * sizeof(int32_t));
+  return 0;
+}
+
+// `bytes` of a call's input to the device, through the staging memory (free:
+// every call that stages an input waits for the stream before it returns).
+int stage_input(hk_engine* e, void* dst, const void* src, size_t bytes) {
+  std::memcpy(e->stage + e->stage_inputs, src, bytes);
+  HK_CHECK(hipMemcpyAsync(dst, e->stage + e->stage_inputs, bytes, hipMemcpyHostToDevice, e->stream));
   return 0;
 }
 
@@ -919,7 +983,10 @@ int hk_engine_create(const hk_model_desc* desc, const hk_model_weights* weights,
     HK_TRY(dalloc(&e->act, d.intermediate));
     HK_TRY(dalloc(&e->normed, d.hidden));
     // the tail past vocab is the persistent step's per-wave store sink
-    HK_TRY(dalloc(&e->logits, (size_t)d.vocab + kPersistentGrid * (kPersistentThreads / 64)));
+    HK_TRY(dalloc(&e->out_block, kOutHead + (size_t)d.vocab + kPersistentGrid * (kPersistentThreads / 64)));
+    e->result = reinterpret_cast<int32_t*>(e->out_block);
+    e->logits = e->out_block + kOutHead;
+    HK_TRY(host_stage(e));
     const size_t kv = (size_t)d.layers * kv_layer_elems(e);
     HK_TRY(dalloc(&e->kcache, kv));
     HK_TRY(dalloc(&e->vcache, kv));
@@ -931,7 +998,6 @@ int hk_engine_create(const hk_model_desc* desc, const hk_model_weights* weights,
     HK_TRY(dalloc(&e->keys, kMaxPartialKeys));
     HK_TRY(dalloc(&e->ctrl, 1));
     HK_TRY(dalloc(&e->out_tokens, d.max_context));
-    HK_TRY(dalloc(&e->result, 3));
     HK_CHECK(hipMemset(e->kcache, 0, kv * sizeof(uint16_t)));
     HK_CHECK(hipMemset(e->vcache, 0, kv * sizeof(uint16_t)));
     HK_CHECK(hipMemset(e->h, 0, d.hidden * sizeof(uint16_t)));
@@ -1028,20 +1094,15 @@ int hk_engine_step(hk_engine* e, int32_t token, int32_t position, int32_t want_l
     return fail("hk_engine_step: outputs requested without want_logits");
   HK_CHECK(hipSetDevice(e->device));
   if (embedding_host != nullptr) {
-    HK_CHECK(hipMemcpyAsync(e->h, embedding_host, e->d.hidden * sizeof(uint16_t),
-                            hipMemcpyHostToDevice, e->stream));
+    HK_TRY(stage_input(e, e->h, embedding_host, e->d.hidden * sizeof(uint16_t)));
     HK_TRY(set_ctrl(e, -1, position, 0));
   } else {
     HK_TRY(set_ctrl(e, token, position, 0));
   }
   HK_TRY(run_step(e, want_logits != 0));
-  if (logits_host)
-    HK_CHECK(hipMemcpyAsync(logits_host, e->logits, (size_t)e->d.vocab * sizeof(float),
-                            hipMemcpyDeviceToHost, e->stream));
   if (embedding_host || logits_host || next_token_host) {
-    int32_t result[2] = {0, 0};
-    HK_CHECK(hipMemcpyAsync(result, e->result, sizeof(result), hipMemcpyDeviceToHost, e->stream));
-    HK_CHECK(hipStreamSynchronize(e->stream));
+    int32_t result[3] = {0, 0, 0};
+    HK_TRY(fetch_outputs(e, result, logits_host));
     HK_TRY(check_persistent(e, result));
     if (next_token_host) *next_token_host = result[0];
   }
@@ -1063,11 +1124,8 @@ int hk_engine_generate(hk_engine* e, int32_t token, int32_t position, int32_t n_
     HK_TRY(run_step(e, true));
   }
   e->next_pos = position + n_steps;
-  int32_t result[2] = {0, 0};
-  HK_CHECK(hipMemcpyAsync(tokens_host, e->out_tokens, (size_t)n_steps * sizeof(int32_t),
-                          hipMemcpyDeviceToHost, e->stream));
-  HK_CHECK(hipMemcpyAsync(result, e->result, sizeof(result), hipMemcpyDeviceToHost, e->stream));
-  HK_CHECK(hipStreamSynchronize(e->stream));
+  int32_t result[3] = {0, 0, 0};
+  HK_TRY(fetch_outputs(e, result, nullptr, tokens_host, n_steps));
   return check_persistent(e, result);
 }
 
@@ -1094,8 +1152,8 @@ int hk_engine_prefill(hk_engine* e, const int32_t* tokens_host, int32_t n, int32
     for (int c0 = 0; c0 < n; c0 += e->pf_rows) {
       const int m = std::min(e->pf_rows, n - c0);
       HK_TRY(m <= kSlabMaxTokens ? native_copies(e) : wide_copies(e));
-      HK_CHECK(hipMemcpyAsync(e->pf_tokens, tokens_host + c0, m * sizeof(int32_t),
-                              hipMemcpyHostToDevice, e->stream));
+      if (c0 > 0) HK_CHECK(hipStreamSynchronize(e->stream));  // pf_tokens and its staging are free again
+      HK_TRY(stage_input(e, e->pf_tokens, tokens_host + c0, m * sizeof(int32_t)));
       HK_TRY(prefill_chunk(e, e->pf_tokens, m, start + c0));
       if (c0 + m == n && want) {
         if (m <= kSlabMaxTokens && e->d.hidden <= kSlabNormMaxK)  // k-blocked x: 16-byte pieces m * 16 bytes apart
@@ -1107,15 +1165,10 @@ int hk_engine_prefill(hk_engine* e, const int32_t* tokens_host, int32_t n, int32
         HK_TRY(set_ctrl(e, -1, start + n - 1, 0));
         HK_TRY(launch_part(e, HK_PART_HEAD, 0));
       }
-      HK_CHECK(hipStreamSynchronize(e->stream));  // pf_tokens is reused by the next chunk
     }
   }
-  if (logits_host)
-    HK_CHECK(hipMemcpyAsync(logits_host, e->logits, (size_t)e->d.vocab * sizeof(float),
-                            hipMemcpyDeviceToHost, e->stream));
   int32_t result[3] = {0, 0, 0};  // token, (step error), split-slab error
-  HK_CHECK(hipMemcpyAsync(result, e->result, sizeof(result), hipMemcpyDeviceToHost, e->stream));
-  HK_CHECK(hipStreamSynchronize(e->stream));
+  HK_TRY(fetch_outputs(e, result, logits_host));
   if (result[2] != 0) {
     // a K-split slab waited too long for one of its parts: this prefill's KV
     // slots and logits are invalid; later prefills run the slabs unsplit

@@ -386,11 +386,14 @@ inline uint16_t host_bf16(float v) {
 
 // `rows` float32 rows of `cols` values, `src_stride` apart, as bf16 rows of
 // padded(cols) values with zeros after the last column.
-void pack_inputs(const float* src, int rows, int cols, size_t src_stride, std::vector<uint16_t>& out) {
+void pack_inputs(const float* src, int rows, int cols, size_t src_stride, uint16_t* out) {
   const int ld = padded(cols);
-  out.assign((size_t)rows * ld, 0);
-  for (int r = 0; r < rows; ++r)
-    for (int c = 0; c < cols; ++c) out[(size_t)r * ld + c] = host_bf16(src[r * src_stride + c]);
+  for (int r = 0; r < rows; ++r) {
+    uint16_t* o = out + (size_t)r * ld;
+    const float* in = src + r * src_stride;
+    for (int c = 0; c < cols; ++c) o[c] = host_bf16(in[c]);
+    for (int c = cols; c < ld; ++c) o[c] = 0;
+  }
 }
 
 // Element (row, col) of a weight tensor in Colibri's upload formats
@@ -449,6 +452,37 @@ struct Scratch {
   }
 };
 
+// Host staging of a call's packed inputs and results, grown on demand: pinned,
+// so that the input copy is queued with the launch, the kernel stores its
+// results straight to the host and one wait ends the call (46 us per 8 x 2048
+// x 2048 Q4_K call with pageable copies, which wait each; 37 with pinned ones
+// both ways; 27 so), or pageable where no pinned memory is to be had.
+struct HostStage {
+  char* buf = nullptr;
+  size_t bytes = 0;
+  bool pinned = false;
+  int reserve(size_t n) {
+    if (n <= bytes) return 0;
+    release();
+    pinned = hipHostMalloc(reinterpret_cast<void**>(&buf), n, hipHostMallocDefault) == hipSuccess;
+    if (!pinned) {
+      (void)hipGetLastError();
+      buf = static_cast<char*>(std::malloc(n));
+      if (!buf) return fail("expert staging: no host memory");
+    }
+    bytes = n;
+    return 0;
+  }
+  void release() {
+    if (buf && pinned)
+      (void)hipHostFree(buf);
+    else
+      std::free(buf);
+    buf = nullptr;
+    bytes = 0;
+  }
+};
+
 inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 }  // namespace
@@ -474,7 +508,7 @@ struct hk_ggml_experts {
   const uint16_t* last_x = nullptr;  // the last call's device input and output,
   float* last_y = nullptr;           // for hk_ggml_mul_mat_id_repeat
   int last_slots = 0, last_input_rows = 0;
-  std::vector<uint16_t> staging;
+  HostStage stage;          // the same on the host
   std::mutex mu;
 };
 
@@ -524,16 +558,30 @@ int run_set(hk_ggml_experts* set, const float* input, int input_rows, const int3
   if (int rc = set->scratch.reserve(in_bytes + out_floats * sizeof(float))) return rc;
   auto* dx = reinterpret_cast<uint16_t*>(set->scratch.buf);
   auto* dy = reinterpret_cast<float*>(set->scratch.buf + in_bytes);
-  pack_inputs(input, input_rows, (int)set->in, set->in, set->staging);
-  hipError_t err = hipMemcpy(dx, set->staging.data(), set->staging.size() * 2, hipMemcpyHostToDevice);
+  if (int rc = set->stage.reserve(in_bytes + out_floats * sizeof(float))) return rc;
+  pack_inputs(input, input_rows, (int)set->in, set->in, reinterpret_cast<uint16_t*>(set->stage.buf));
+  hipError_t err = hipMemcpyAsync(dx, set->stage.buf, (size_t)input_rows * set->ld * 2, hipMemcpyHostToDevice, nullptr);
   if (err != hipSuccess) return hip_fail(err, "expert input copy");
-  if (int rc = launch_set(set, ids, n, input_rows, dx, dy)) return rc;
+  auto* results = reinterpret_cast<float*>(set->stage.buf + in_bytes);
+  if (int rc = launch_set(set, ids, n, input_rows, dx, set->stage.pinned ? results : dy)) return rc;
   set->last_x = dx;
   set->last_y = dy;
   set->last_slots = n;
   set->last_input_rows = input_rows;
-  err = hipMemcpy(out, dy, out_floats * sizeof(float), hipMemcpyDeviceToHost);
-  return err == hipSuccess ? HK_OK : hip_fail(err, "expert output copy");
+  if (!set->stage.pinned) err = hipMemcpyAsync(results, dy, out_floats * sizeof(float), hipMemcpyDeviceToHost, nullptr);
+  if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
+  if (err != hipSuccess) return hip_fail(err, "expert output copy");
+  std::memcpy(out, results, out_floats * sizeof(float));
+  return HK_OK;
+}
+
+// The scratch and staging of a set's largest ordinary call, at its creation
+// (a call reserves again what could not be had).
+void reserve_call(hk_ggml_experts* set) {
+  const size_t rows = set->kind == kW8Tile || set->experts == 1 ? 1 : kGroupMax;
+  const size_t bytes = align256(rows * set->ld * 2) + rows * set->out * sizeof(float);
+  (void)set->scratch.reserve(bytes);
+  (void)set->stage.reserve(bytes);
 }
 
 // Q6_K blocks of one expert ([out][nb][210]) as planes (see QArgs).
@@ -600,6 +648,7 @@ int hk_ggml_experts_create(const float* weights, int64_t n_experts, int64_t out_
     hk_ggml_experts_destroy(set);
     return hip_fail(err, "hk_ggml_experts_create");
   }
+  reserve_call(set);
   *out = set;
   return HK_OK;
 }
@@ -639,6 +688,7 @@ int hk_ggml_dense_create(const float* weights, int64_t out_dim, int64_t in_dim, 
     hk_ggml_experts_destroy(set);
     return hip_fail(err, "hk_ggml_dense_create");
   }
+  reserve_call(set);
   *out = set;
   return HK_OK;
 }
@@ -674,6 +724,7 @@ int hk_ggml_quant_create(int ggml_type, const void* blocks, int64_t n_experts, i
     hk_ggml_experts_destroy(set);
     return hip_fail(err, "hk_ggml_quant_create");
   }
+  reserve_call(set);
   *out = set;
   return HK_OK;
 }
@@ -762,6 +813,7 @@ void hk_ggml_experts_destroy(hk_ggml_experts* set) {
   if (set->s) (void)hipFree(set->s);
   if (set->blocks) (void)hipFree(set->blocks);
   set->scratch.release();
+  set->stage.release();
   delete set;
 }
 
@@ -780,7 +832,7 @@ namespace {
 struct ColiRuntime {
   std::atomic<bool> up{false};
   Scratch scratch;
-  std::vector<uint16_t> staging;
+  HostStage stage;
   std::mutex mu;
 };
 
@@ -802,18 +854,40 @@ bool coli_pack(ColiCudaTensor* t, const void* weights, const float* scales) {
          hipMemcpy(t->s, s.data(), s.size() * sizeof(float), hipMemcpyHostToDevice) == hipSuccess;
 }
 
-// Copies `rows` float32 input rows (back to back) into the scratch as padded
-// bf16 rows, reserving `extra_bytes` after them (returned in *rest); returns
-// the rows' device address, or null on failure.  Holds coli().mu.
-uint16_t* coli_stage_inputs(const float* input, int rows, int cols, size_t extra_bytes, char** rest) {
+// Queues the copy of `rows` float32 input rows (back to back) into the scratch
+// as padded bf16 rows, reserving `extra_bytes` after them (returned in *rest)
+// and `out_floats` for coli_results; returns the rows' device address, or null
+// on failure.  Holds coli().mu.
+uint16_t* coli_stage_inputs(const float* input, int rows, int cols, size_t extra_bytes, size_t out_floats,
+                            char** rest) {
   ColiRuntime& rt = coli();
-  const size_t in_bytes = align256((size_t)rows * padded(cols) * 2);
+  const size_t copied = (size_t)rows * padded(cols) * 2, in_bytes = align256(copied);
   if (rt.scratch.reserve(in_bytes + extra_bytes)) return nullptr;
-  pack_inputs(input, rows, cols, cols, rt.staging);
-  if (hipMemcpy(rt.scratch.buf, rt.staging.data(), rt.staging.size() * 2, hipMemcpyHostToDevice) != hipSuccess)
+  if (rt.stage.reserve(in_bytes + out_floats * sizeof(float))) return nullptr;
+  pack_inputs(input, rows, cols, cols, reinterpret_cast<uint16_t*>(rt.stage.buf));
+  if (hipMemcpyAsync(rt.scratch.buf, rt.stage.buf, copied, hipMemcpyHostToDevice, nullptr) != hipSuccess)
     return nullptr;
   *rest = rt.scratch.buf + in_bytes;
   return reinterpret_cast<uint16_t*>(rt.scratch.buf);
+}
+
+// Where the call's kernel stores its `n` result floats: the last of the staging
+// (after the inputs), or dy where that is no pinned memory.
+float* coli_target(float* dy, size_t n) {
+  ColiRuntime& rt = coli();
+  return rt.stage.pinned ? reinterpret_cast<float*>(rt.stage.buf + rt.stage.bytes) - n : dy;
+}
+
+// Waits for the call and hands its results to the caller.
+int coli_results(const float* dy, size_t n, float* output) {
+  ColiRuntime& rt = coli();
+  float* results = reinterpret_cast<float*>(rt.stage.buf + rt.stage.bytes) - n;
+  if (!rt.stage.pinned &&
+      hipMemcpyAsync(results, dy, n * sizeof(float), hipMemcpyDeviceToHost, nullptr) != hipSuccess)
+    return 0;
+  if (hipStreamSynchronize(nullptr) != hipSuccess) return 0;
+  std::memcpy(output, results, n * sizeof(float));
+  return 1;
 }
 
 }  // namespace
@@ -831,6 +905,7 @@ int coli_cuda_init(const int* devices, int count) {
 void coli_cuda_shutdown(void) {
   std::lock_guard<std::mutex> lock(coli().mu);
   coli().scratch.release();
+  coli().stage.release();
   coli().up = false;
 }
 
@@ -893,7 +968,7 @@ int coli_cuda_expert_group_pinned(ColiCudaTensor* const* gate, ColiCudaTensor* c
   std::lock_guard<std::mutex> lock(coli().mu);
   const size_t act_bytes = align256((size_t)count * ld_mid * 2), ny = (size_t)count * in;
   char* rest = nullptr;
-  uint16_t* dx = coli_stage_inputs(input, count, in, act_bytes + ny * sizeof(float), &rest);
+  uint16_t* dx = coli_stage_inputs(input, count, in, act_bytes + ny * sizeof(float), ny, &rest);
   if (!dx) return 0;
   auto* dact = reinterpret_cast<uint16_t*>(rest);
   auto* dy = reinterpret_cast<float*>(rest + act_bytes);
@@ -921,10 +996,10 @@ int coli_cuda_expert_group_pinned(ColiCudaTensor* const* gate, ColiCudaTensor* c
     b.q[i] = down[i]->q;
     b.s[i] = down[i]->s;
     b.x[i] = dact + (size_t)i * ld_mid;
-    b.y[i] = dy + (size_t)i * in;
+    b.y[i] = coli_target(dy, ny) + (size_t)i * in;
   }
   if (launch_experts(b, count, false, nullptr)) return 0;
-  return hipMemcpy(output, dy, ny * sizeof(float), hipMemcpyDeviceToHost) == hipSuccess ? 1 : 0;
+  return coli_results(dy, ny, output);
 }
 
 int coli_cuda_expert_group(ColiCudaTensor* const* gate, ColiCudaTensor* const* up, ColiCudaTensor* const* down,
@@ -951,7 +1026,7 @@ int coli_cuda_matmul(ColiCudaTensor** tensor, float* output, const float* input,
   if (!coli().up) return 0;
   std::lock_guard<std::mutex> lock(coli().mu);
   char* rest = nullptr;
-  uint16_t* dx = coli_stage_inputs(input, 1, t->input, (size_t)t->output * sizeof(float), &rest);
+  uint16_t* dx = coli_stage_inputs(input, 1, t->input, (size_t)t->output * sizeof(float), t->output, &rest);
   if (!dx) return 0;
   auto* dy = reinterpret_cast<float*>(rest);
   ExpertArgs a{};
@@ -962,9 +1037,9 @@ int coli_cuda_matmul(ColiCudaTensor** tensor, float* output, const float* input,
   a.q[0] = t->q;
   a.s[0] = t->s;
   a.x[0] = dx;
-  a.y[0] = dy;
+  a.y[0] = coli_target(dy, t->output);
   if (launch_experts(a, 1, false, nullptr)) return 0;
-  return hipMemcpy(output, dy, (size_t)t->output * sizeof(float), hipMemcpyDeviceToHost) == hipSuccess ? 1 : 0;
+  return coli_results(dy, t->output, output);
 }
 
 }  // extern "C"

@@ -138,7 +138,6 @@ class QwenDecoderEngine:
             "hk_engine_create",
         )
         self._engine = handle.value
-        self._logits = np.empty(self.vocab, dtype=np.float32)
         self._token = ctypes.c_int32()
 
     def _upload(self, array):
@@ -183,7 +182,7 @@ class QwenDecoderEngine:
         row = np.ascontiguousarray(np.asarray(embedding, dtype=np.uint16))
         if row.shape != (self.hidden,):
             raise ValueError(f"embedding row must have {self.hidden} bf16 values")
-        out = self._logits if logits else None
+        out = np.empty(self.vocab, dtype=np.float32) if logits else None
         hip.check(
             self._lib.hk_engine_step(
                 self._live(), 0, int(position), 1 if logits else 0, row.ctypes.data,
@@ -191,7 +190,7 @@ class QwenDecoderEngine:
             ),
             "hk_engine_step",
         )
-        return np.array(out, copy=True) if logits else None
+        return out
 
     def step_token(self, token_id, position, logits=True, want_logits_array=True):
         """Like ``step`` but the embedding row is looked up on the device.
@@ -203,7 +202,7 @@ class QwenDecoderEngine:
                 "hk_engine_step",
             )
             return None, None
-        out = self._logits if want_logits_array else None
+        out = np.empty(self.vocab, dtype=np.float32) if want_logits_array else None
         hip.check(
             self._lib.hk_engine_step(
                 self._live(), int(token_id), int(position), 1, None,
@@ -211,7 +210,7 @@ class QwenDecoderEngine:
             ),
             "hk_engine_step",
         )
-        return int(self._token.value), (np.array(out, copy=True) if out is not None else None)
+        return int(self._token.value), out
 
     def prefill(self, token_ids, start=0, logits=True, want_logits_array=True):
         """All prompt tokens at slots start..start+n-1 in one batched pass
@@ -220,7 +219,7 @@ class QwenDecoderEngine:
         ids = np.ascontiguousarray(np.asarray(token_ids, dtype=np.int32))
         if ids.ndim != 1 or ids.size == 0:
             raise ValueError("prefill needs a non-empty 1-D list of token ids")
-        out = self._logits if (logits and want_logits_array) else None
+        out = np.empty(self.vocab, dtype=np.float32) if (logits and want_logits_array) else None
         hip.check(
             self._lib.hk_engine_prefill(
                 self._live(), ids.ctypes.data, int(ids.size), int(start),
@@ -231,7 +230,7 @@ class QwenDecoderEngine:
         )
         if not logits:
             return None, None
-        return int(self._token.value), (np.array(out, copy=True) if out is not None else None)
+        return int(self._token.value), out
 
     def generate(self, token_id, position, n_steps):
         """Greedy decode: ``n_steps`` tokens starting from ``token_id`` at
