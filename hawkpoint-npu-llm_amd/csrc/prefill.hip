@@ -19,6 +19,7 @@
 // SwiGLU pairs), each wave a 32x32 quarter as 2x2 MFMA 16x16x32 blocks; K
 // advances 32 at a time through LDS.
 #include <algorithm>
+#include <type_traits>
 
 #include "hk_common.h"
 #include "hk_internal.h"
@@ -445,6 +446,14 @@ __device__ __forceinline__ void lds_ready(bf16x8& v) {
 #endif
 }
 
+// Waits until at most N of the wave's LDS reads are outstanding.
+template <int N>
+__device__ __forceinline__ void lds_wait() {
+  static_assert(N >= 0 && N <= 15, "a four-bit counter");
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (N << 8));
+  asm volatile("" ::: "memory");
+}
+
 template <int BM, int BN, bool PAIR, int NS, int RK, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring_kernel(PrefillGemmArgs a) {
   constexpr int WR = PAIR ? 2 * BN : BN;  // weight rows per tile
@@ -554,28 +563,37 @@ __global__ __launch_bounds__(kThreads, PAIR && BN == 128 ? 2 : 1) void gemm_ring
         if constexpr (PAIR) uf[h][j] = lds_read16(ws + (BN + wn + 32 * j + fr) * RK + pos[h]);
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    // (the products take the fragments from here on: after the wait)
+    // each 16-deep step's products start once its own fragments are there: LDS
+    // answers in order, so the later steps' reads may still be in flight (one
+    // wait for all of them had the 64 x 64 tiles 2-4% slower); the waves of the
+    // largest tiles hold their issue slot over a step's products (1-3%)
+    auto products = [&](auto step) {
+      constexpr int h = decltype(step)::value;
+      if constexpr (h < NH) {
+        lds_wait<(NH - 1 - h) * (MB + (PAIR ? 2 : 1) * NB)>();
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-#pragma unroll
-      for (int i = 0; i < MB; ++i) lds_ready(af[h][i]);
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        lds_ready(bf[h][j]);
-        if constexpr (PAIR) lds_ready(uf[h][j]);
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < NH; ++h)
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
+        for (int i = 0; i < MB; ++i) lds_ready(af[h][i]);
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[h][i], bf[h][j], acc[i][j], 0, 0, 0);
-          if constexpr (PAIR)
-            accu[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[h][i], uf[h][j], accu[i][j], 0, 0, 0);
+          lds_ready(bf[h][j]);
+          if constexpr (PAIR) lds_ready(uf[h][j]);
         }
+        if constexpr (BM * BN == 128 * 128) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[h][i], bf[h][j], acc[i][j], 0, 0, 0);
+            if constexpr (PAIR)
+              accu[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[h][i], uf[h][j], accu[i][j], 0, 0, 0);
+          }
+        if constexpr (BM * BN == 128 * 128) __builtin_amdgcn_s_setprio(0);
+      }
+    };
+    products(std::integral_constant<int, 0>{});
+    products(std::integral_constant<int, 1>{});
+    products(std::integral_constant<int, 2>{});
+    products(std::integral_constant<int, 3>{});
   }
   if constexpr (SPLIT) {
     // lane holds rows 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
@@ -1573,12 +1591,12 @@ int launch_ring(const PrefillGemmArgs& args, hipStream_t stream, bool* normed) {
     else
       launch_ring_tiles<64, 64, false, 4, 32>(a, stream);
   } else if (pair) {
-    // gate/up in 128 x (64 + 64) tiles, three per CU, while they run at once
-    // (417 tokens 19.6 against 25.7 us in the larger ones, 1021 31.8 and
-    // 33.9); then 128 x (128 + 128) ones, each wave 64 tokens x 64 gate + 64
-    // up outputs at two waves per SIMD (1500 tokens 38.8 against 40.3, 4064
-    // 82.6 and 84.7)
-    if (tiles_of(a.M, a.N, 128, 64) <= 3 * cu_count())
+    // gate/up in 128 x (64 + 64) tiles, three workgroups per CU, for up to two
+    // rounds of them, then 128 x (128 + 128) ones, two per CU with each wave 64
+    // tokens x 64 gate + 64 up outputs (417 tokens 20.0 and 26.4 us, 1021 32.1
+    // and 34.9, 2048 47.6 and 56.8; a 4064-token prefill of four layers 1259
+    // and 1250)
+    if (tiles_of(a.M, a.N, 128, 64) <= 6 * cu_count())
       launch_ring_tiles<128, 64, true, 3, 32>(a, stream);
     else
       launch_ring_tiles<128, 128, true, 3, 32>(a, stream);
