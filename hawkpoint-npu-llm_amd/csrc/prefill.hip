@@ -1454,11 +1454,14 @@ int tiles_of(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + 
 // CU beyond, every part at least twelve 64-deep stages.  down_proj (K 4864,
 // N 896), us with the parts taken and unsplit or with one part fewer: 65
 // tokens 10.6 (6), 256 12.2 (4) and 13.4 (3), 417 15.0 (4) and 16.0 (3), 1021
-// 22.6 (2) and 23.2 (1).
+// 22.6 (2) and 23.2 (1).  A shorter K is split in two where that leaves the
+// RMSNorm after it to the second pass: O (K 896) and the norm, 100 tokens 7.4
+// against 6.9 + 3.5, 417 8.6 against 6.9 + 3.8, 1021 11.5 against 7.2 + 5.0.
 int ring_parts(int M, int N, int K) {
   const int t = tiles_of(M, N, 64, 64), stages = K / 64;
   if (t > 448 || N % 8 != 0) return 1;
-  const int want = std::max(1, std::min({6, (t <= 64 ? 256 : 448) / t, stages / 12}));
+  const int most = t <= 224 && stages >= 8 ? std::max(2, stages / 12) : stages / 12;
+  const int want = std::max(1, std::min({6, (t <= 64 ? 256 : 448) / t, most}));
   const int per = (stages + want - 1) / std::max(want, 1);
   return per > 0 ? (stages + per - 1) / per : 1;
 }
