@@ -215,6 +215,8 @@ struct hk_engine {
   int32_t* pf_tokens = nullptr;
   float* pf_split = nullptr;   // split-K partial sums of GEMMs with few tiles
   size_t pf_split_floats = 0;
+  float* pf_attn_parts = nullptr;      // PrefillAttnArgs::part_ws
+  unsigned* pf_attn_tickets = nullptr;
   // per layer, MFMA-native copies of qkv (RoPE order), o, gate_up and down
   // for the slab GEMMs of chunks up to 64 tokens (empty: row-major weights)
   std::vector<std::array<void*, 4>> pf_native;
@@ -492,7 +494,7 @@ void free_engine(hk_engine* e) {
                   e->counters, e->keys,    e->ctrl,     e->out_tokens,
                   e->pf_x,    e->pf_h1,    e->pf_xn,    e->pf_qkv,     e->pf_q,
                   e->pf_att,  e->pf_act,   e->pf_tokens, e->pf_split, e->players, e->psync, e->ptag,
-                  e->wpart,   e->xpart, e->pf_wide};
+                  e->wpart,   e->xpart, e->pf_wide, e->pf_attn_parts, e->pf_attn_tickets};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (uint16_t* p : e->down_x)
@@ -575,6 +577,7 @@ void free_prefill_buffers(hk_engine* e) {
   };
   drop(e->pf_x), drop(e->pf_h1), drop(e->pf_xn), drop(e->pf_qkv), drop(e->pf_q);
   drop(e->pf_att), drop(e->pf_act), drop(e->pf_tokens), drop(e->pf_split), drop(e->slab_ws);
+  drop(e->pf_attn_parts), drop(e->pf_attn_tickets);
   e->pf_rows = 0;
 }
 
@@ -596,6 +599,9 @@ int alloc_prefill_buffers(hk_engine* e, int rows) {
     e->pf_split_floats = std::max({e->pf_split_floats, split_ws_need(m, d.hidden, QD),
                                    split_ws_need(m, d.hidden, d.intermediate)});
   HK_TRY(dalloc(&e->pf_split, e->pf_split_floats));
+  HK_TRY(dalloc(&e->pf_attn_parts, attn_part_floats()));
+  HK_TRY(dalloc(&e->pf_attn_tickets, kAttnMaxTasks));
+  HK_CHECK(hipMemset(e->pf_attn_tickets, 0, kAttnMaxTasks * sizeof(unsigned)));
   // tagged partial sums of the K-split down slabs (N = hidden); tag 0 never
   // matches a launch's
   const size_t slab_words = (size_t)((d.hidden + 15) / 16) * kSlabParts * kSlabMaxTokens * 16;
@@ -765,6 +771,8 @@ int prefill_chunk(hk_engine* e, const int32_t* tokens_dev, int n, int start) {
     at.out = e->pf_att;
     at.ld_out = QD;
     at.out_kblock = kb;
+    at.part_ws = e->pf_attn_parts;
+    at.tickets = e->pf_attn_tickets;
     at.rope_done = rope_fused ? 1 : 0;
     at.n = n;
     at.start = start;

@@ -285,8 +285,16 @@ struct PrefillAttnArgs {
   int out_kblock;           // nonzero: out k-blocked with n rows (see PrefillGemmArgs::kblock)
   int rope_done;            // nonzero: qrot and the caches are written already (the QKV GEMM's RoPE)
   int n, start, q_heads, kv_heads, max_ctx;
-  int period;               // set by launch_prefill_attention: the CU count
+  // Optional: partial results of tasks whose KV blocks are split over
+  // workgroups (attn_part_floats() floats) and a zeroed ticket per task
+  // (kAttnMaxTasks)
+  float* part_ws;
+  unsigned* tickets;
+  int period, parts;        // set by launch_prefill_attention: the CU count, KV parts per task
 };
+constexpr int kAttnPartSlots = 512;  // workgroups of a split launch at most
+constexpr int kAttnMaxTasks = 256;
+size_t attn_part_floats();
 
 // Whether a QKV GEMM of more than 64 tokens can apply RoPE and the KV append
 // in its epilogue (PrefillGemmArgs::rope).

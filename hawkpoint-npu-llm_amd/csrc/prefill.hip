@@ -1229,7 +1229,15 @@ __device__ __forceinline__ float quad_sum(float v) {
 // forms give the same result).  With up to 128 VGPRs (four waves per SIMD
 // for ST > 1, at least two for ST = 1) the compiler keeps the MFMA sums in
 // VGPRs; in AGPRs every score and every rescale of O cost extra moves.
-template <int KS, int ST>
+//
+// SPLIT: few tasks over a long context (a chat's next turn over its cached
+// history).  The KV blocks of a task go to up to a.parts workgroups, in runs;
+// each leaves its (max, sum, O) in a.part_ws with device-coherent stores, and
+// the last of a task to finish (a ticket per task, zero between launches)
+// folds the parts in part order.  40 tokens at slot 3000 (14 tasks of 24
+// blocks): 22 us per layer less than with a workgroup per task.
+constexpr int kPartFloats = 20;  // per lead thread and part: O (16), max, sum, 2 unused
+template <int KS, int ST, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_prefill_kernel(PrefillAttnArgs a) {
   constexpr int kSB = KS / 16;  // 16-slot S^T blocks per KV block
   static_assert(KS == 64 || KS == kFaSlots, "64 or kFaSlots slots per block");
@@ -1244,7 +1252,7 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
   const int nblk = (a.n + kFaRows - 1) / kFaRows, tasks = nblk * a.q_heads;
   const int run = (int)blockIdx.x / a.period, pos = (int)blockIdx.x % a.period;
   const int run_len = min(a.period, tasks - run * a.period);
-  const int rank = run * a.period + ((run & 1) ? run_len - 1 - pos : pos);
+  const int rank = SPLIT ? (int)blockIdx.x % tasks : run * a.period + ((run & 1) ? run_len - 1 - pos : pos);
   const int h = rank % a.q_heads;
   const int qb = nblk - 1 - rank / a.q_heads;
   const int g = h / (a.q_heads / a.kv_heads);
@@ -1256,7 +1264,11 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
   const int p = a.start + (tok_ok ? tok : 0);
   const int last_slot = a.start + min(qb * kFaRows + kFaRows - 1, a.n - 1);
   const int nkv = last_slot / KS + 1;
-  const int iters = (nkv + ST - 1) / ST;  // rounds of ST blocks
+  // this workgroup's blocks [kb0, kb1): all of them, or a part's run
+  const int per_part = SPLIT ? (nkv + a.parts - 1) / a.parts : nkv, part = SPLIT ? (int)blockIdx.x / tasks : 0;
+  const int kb0 = part * per_part, kb1 = min(nkv, kb0 + per_part);
+  if (SPLIT && kb0 >= kb1) return;  // (fewer runs than parts)
+  const int iters = (kb1 - kb0 + ST - 1) / ST;  // rounds of ST blocks
   const size_t kv_base = (size_t)g * a.max_ctx;
   const u32x4 zero = {0u, 0u, 0u, 0u};
 
@@ -1281,7 +1293,7 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
   u32x4 kr[kLoads], vr[kLoads];
   auto load_tile = [&](int kb) {
     // (a block past the last has no slot: its offsets lie past the resources)
-    const unsigned off = kb < nkv ? (unsigned)((kb * KS + ls) * kHeadDim + ld0) * 2u : 0x7ffffff0u;
+    const unsigned off = kb < kb1 ? (unsigned)((kb * KS + ls) * kHeadDim + ld0) * 2u : 0x7ffffff0u;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       kr[i] = __builtin_amdgcn_raw_buffer_load_b128(kres, off, 32 * kHeadDim * 2 * i, 0);
@@ -1293,9 +1305,9 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
   f32x4 o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  load_tile(stream);
+  load_tile(kb0 + stream);
   for (int it = 0; it < iters; ++it) {
-    const int kb = it * ST + stream;
+    const int kb = kb0 + it * ST + stream;
     __syncthreads();  // the previous tiles have been read
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
@@ -1304,7 +1316,7 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
     }
     __syncthreads();
     if (it + 1 < iters) load_tile(kb + ST);  // in flight during this tile's math
-    if (kb >= nkv) continue;  // this stream's final round holds no block (uniform per stream)
+    if (kb >= kb1) continue;  // this stream's final round holds no block (uniform per stream)
 
     // S^T blocks: lane holds slots s0 + 16 sb + 4 quad + r of token `tok`
     const int s0 = kb * KS;
@@ -1416,10 +1428,10 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
         for (int r = 0; r < 4; ++r) d[2 + 4 * db + r] = o[db][r];
     }
     __syncthreads();
-    if (stream > 0) return;
+    if (!SPLIT && stream > 0) return;
 #pragma unroll
     for (int q = 1; q < ST; ++q) {
-      const float* d = xs + (((q - 1) * 4 + sw) * 64 + lane) * kW;
+      const float* d = xs + (((q - 1) * 4 + sw) * 64 + lane) * kW;  // (SPLIT: only stream 0's fold is used)
       const float mq = d[0];
       const float m_new = fmaxf(m_run, mq);
       const float m_use = m_new == -INFINITY ? 0.0f : m_new;
@@ -1431,6 +1443,51 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
         for (int r = 0; r < 4; ++r) o[db][r] = o[db][r] * a0 + d[2 + 4 * db + r] * a1;
       m_run = m_new;
     }
+  }
+  if constexpr (SPLIT) {
+    __shared__ int last;
+    const int runs = (nkv + per_part - 1) / per_part;  // parts of this task that have blocks
+    constexpr int kSc1 = 16;                           // device-coherent
+    const __amdgpu_buffer_rsrc_t ws =
+        rsrc(a.part_ws + (size_t)rank * a.parts * kThreads * kPartFloats, a.parts * kThreads * kPartFloats * 4);
+    const unsigned mine = (unsigned)stid * (kPartFloats * 4), stride = kThreads * kPartFloats * 4;
+    if (stream == 0) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[db]), ws, mine + part * stride + 16 * db, 0,
+                                               kSc1);
+      const u32x2_t ml = {__float_as_uint(m_run), __float_as_uint(l_run)};
+      __builtin_amdgcn_raw_buffer_store_b64(ml, ws, mine + part * stride + 64, 0, kSc1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __syncthreads();  // every wave's stores have completed
+    if (tid == 0)
+      last = __hip_atomic_fetch_add(&a.tickets[rank], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(runs - 1);
+    __syncthreads();
+    if (!last || stream > 0) return;
+    m_run = -INFINITY;
+    for (int q = 0; q < runs; ++q) {
+      const u32x2_t ml = __builtin_amdgcn_raw_buffer_load_b64(ws, mine + q * stride + 64, 0, kSc1);
+      m_run = fmaxf(m_run, __uint_as_float(ml.x));
+    }
+    const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+    l_run = 0.0f;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int q = 0; q < runs; ++q) {
+      const u32x2_t ml = __builtin_amdgcn_raw_buffer_load_b64(ws, mine + q * stride + 64, 0, kSc1);
+      const float f = __builtin_amdgcn_exp2f(__uint_as_float(ml.x) - m_use);
+      l_run = fmaf(__uint_as_float(ml.y), f, l_run);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const f32x4 po = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, mine + q * stride + 16 * db, 0, kSc1));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[db][r] = fmaf(po[r], f, o[db][r]);
+      }
+    }
+    if (tid == 0) __hip_atomic_store(&a.tickets[rank], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!tok_ok) return;
 #pragma unroll
@@ -1711,6 +1768,23 @@ int launch_rmsnorm_rows(const uint16_t* X, int ldx, const uint16_t* gamma, float
   return err == hipSuccess ? 0 : hip_fail(err, "rmsnorm rows launch");
 }
 
+size_t attn_part_floats() { return (size_t)kAttnPartSlots * kThreads * kPartFloats; }
+
+namespace {
+// KV parts of the attention's tasks: with at most one task per CU and six or
+// more 128-slot blocks per task (on average: the causal tasks of a prompt from
+// slot 0 see half the context), as many as keep the workgroups within two per
+// CU and give every part two blocks, one round of its two streams.  Four-layer
+// prefills with logits, us with a workgroup per task and split: 40 tokens at
+// slot 1000 324 and 306, at 3000 420 and 330, 200 at 3000 494 and 425, 1000 at
+// 3000 664 and 612; 1021 at 0 (four blocks per task) 510 and 519.
+int attn_parts(const PrefillAttnArgs& a, int tasks) {
+  const int blocks = (2 * a.start + a.n) / (2 * kFaSlots);
+  if (!a.part_ws || blocks < 6 || tasks > kAttnMaxTasks) return 1;
+  return std::max(1, std::min(kAttnPartSlots / tasks, blocks / 2));
+}
+}  // namespace
+
 int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream) {
   if (a.q_heads % a.kv_heads != 0) return fail("prefill attention: unsupported head grouping");
   if (a.ld_out % 4 != 0) return fail("prefill attention: output rows must be 8-byte aligned");
@@ -1726,6 +1800,9 @@ int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream) {
   const dim3 grid(a.q_heads * ((a.n + kFaRows - 1) / kFaRows));
   if (a.start + a.n <= 64)
     hipLaunchKernelGGL((attention_prefill_kernel<64, 1>), grid, dim3(kThreads), 0, stream, b);
+  else if ((b.parts = attn_parts(a, (int)grid.x)) > 1)
+    hipLaunchKernelGGL((attention_prefill_kernel<kFaSlots, kFaStreams, true>), dim3(grid.x * b.parts),
+                       dim3(kThreads * kFaStreams), 0, stream, b);
   else
     hipLaunchKernelGGL((attention_prefill_kernel<kFaSlots, kFaStreams>), grid, dim3(kThreads * kFaStreams), 0,
                        stream, b);

@@ -215,6 +215,34 @@ def test_prefill_continues_from_cached_prefix():
         engine.close()
 
 
+@pytest.mark.parametrize("n,start", [(1, 1300), (40, 767), (65, 800), (200, 1200), (700, 900)])
+def test_prefill_after_a_long_history(n, start):
+    """A chat's next turn over its cached history: few attention tasks over
+    many KV blocks, split over workgroups whose partial results the last one
+    folds (one to eleven tasks per head, parts with one block and with none
+    left), twice so that the tickets are seen to reset; against the oracle."""
+    from runtime.qwen_engine import QwenDecoderEngine
+
+    announce(f"prefill of {n} after {start}")
+    model = SyntheticModel(QWEN25_05B, seed=11, layers=2)
+    prompt = _prompt(151936, start + n, 80 + n)
+    oracle = OracleDecoder(model, 1700)
+    ref_tok, ref = oracle.prefill(prompt)
+    engine = QwenDecoderEngine(model, context_length=1700)
+    try:
+        engine.prefill(prompt[:start], 0, logits=False)
+        tok, logits = engine.prefill(prompt[start:], start)
+        tok2, logits2 = engine.prefill(prompt[start:], start)
+        assert rel_l2(logits, ref) <= 1e-2
+        assert tok == ref_tok or near_tie(ref)
+        assert tok2 == tok
+        np.testing.assert_array_equal(logits2, logits)
+        for slot in (start, start + n - 1):
+            check_kv_slot(engine, oracle.stage, 1, slot, 2e-2)
+    finally:
+        engine.close()
+
+
 @pytest.mark.parametrize("n,w8", [(1, False), (16, False), (17, False), (32, False), (33, False), (48, False),
                                   (49, False), (63, False), (64, False), (65, False), (130, False), (1, True),
                                   (17, True), (40, True), (64, True)])
