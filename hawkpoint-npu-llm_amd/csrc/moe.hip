@@ -192,11 +192,22 @@ __device__ void plan_pairs(PlanLds& l, int T, int K, int E, int S, int max_group
     }
     return v;
   };
-  for (int e = wave; e < E; e += nt / 64) {
-    const int c = lane < W ? __popcll(l.bits[e][lane]) : 0;
-    const int incl = inclusive(c);
-    if (lane < W) l.before[e][lane] = (uint16_t)(incl - c);
-    if (lane == 63) l.counts[e] = incl;
+  if (W <= 8) {  // (small batches: a thread per expert, no scan over lanes)
+    for (int e = tid; e < E; e += nt) {
+      int sum = 0;
+      for (int w = 0; w < W; ++w) {
+        l.before[e][w] = (uint16_t)sum;
+        sum += __popcll(l.bits[e][w]);
+      }
+      l.counts[e] = sum;
+    }
+  } else {
+    for (int e = wave; e < E; e += nt / 64) {
+      const int c = lane < W ? __popcll(l.bits[e][lane]) : 0;
+      const int incl = inclusive(c);
+      if (lane < W) l.before[e][lane] = (uint16_t)(incl - c);
+      if (lane == 63) l.counts[e] = incl;
+    }
   }
   __syncthreads();
   if (wave == 0) {
