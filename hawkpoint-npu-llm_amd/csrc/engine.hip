@@ -181,6 +181,7 @@ struct hk_engine {
   char* stage = nullptr;
   size_t stage_inputs = 0;   // offset of the inputs
   bool stage_pinned = false;
+  bool stage_queued = false;  // the inputs' copy may be in flight
   // whole step in one persistent launch (persistent.hip); -1: per-kernel graph
   int pshape = -1;
   // the step may also run split by XCD (attention block on XCD 0); it does so
@@ -550,15 +551,19 @@ int fetch_outputs(hk_engine* e, int32_t (&result)[3], float* logits_host, int32_
   if (tokens_host)
     HK_CHECK(hipMemcpyAsync(body, e->out_tokens, n_tokens * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
   HK_CHECK(hipStreamSynchronize(e->stream));
+  e->stage_queued = false;
   std::memcpy(result, e->stage, sizeof(result));
   if (logits_host) std::memcpy(logits_host, body, logits);
   if (tokens_host) std::memcpy(tokens_host, body, n_tokens * sizeof(int32_t));
   return 0;
 }
 
-// `bytes` of a call's input to the device, through the staging memory (free:
-// every call that stages an input waits for the stream before it returns).
+// `bytes` of a call's input to the device, through the staging memory: after
+// the copy of the inputs before it, which may still be reading (a prompt's
+// earlier chunk, or a call that failed on the way to fetch_outputs).
 int stage_input(hk_engine* e, void* dst, const void* src, size_t bytes) {
+  if (e->stage_queued) HK_CHECK(hipStreamSynchronize(e->stream));
+  e->stage_queued = true;
   std::memcpy(e->stage + e->stage_inputs, src, bytes);
   HK_CHECK(hipMemcpyAsync(dst, e->stage + e->stage_inputs, bytes, hipMemcpyHostToDevice, e->stream));
   return 0;
@@ -1160,7 +1165,6 @@ int hk_engine_prefill(hk_engine* e, const int32_t* tokens_host, int32_t n, int32
     for (int c0 = 0; c0 < n; c0 += e->pf_rows) {
       const int m = std::min(e->pf_rows, n - c0);
       HK_TRY(m <= kSlabMaxTokens ? native_copies(e) : wide_copies(e));
-      if (c0 > 0) HK_CHECK(hipStreamSynchronize(e->stream));  // pf_tokens and its staging are free again
       HK_TRY(stage_input(e, e->pf_tokens, tokens_host + c0, m * sizeof(int32_t)));
       HK_TRY(prefill_chunk(e, e->pf_tokens, m, start + c0));
       if (c0 + m == n && want) {

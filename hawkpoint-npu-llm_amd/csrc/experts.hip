@@ -461,7 +461,11 @@ struct HostStage {
   char* buf = nullptr;
   size_t bytes = 0;
   bool pinned = false;
+  bool queued = false;  // a call's copies and stores may be in flight
+  // Waits for what an earlier call left in flight (one that failed after its
+  // input copy was queued), then has room for `n` bytes.
   int reserve(size_t n) {
+    if (const hipError_t err = settle(); err != hipSuccess) return hip_fail(err, "expert staging");
     if (n <= bytes) return 0;
     release();
     pinned = hipHostMalloc(reinterpret_cast<void**>(&buf), n, hipHostMallocDefault) == hipSuccess;
@@ -473,7 +477,13 @@ struct HostStage {
     bytes = n;
     return 0;
   }
+  hipError_t settle() {
+    const hipError_t err = queued ? hipStreamSynchronize(nullptr) : hipSuccess;
+    if (err == hipSuccess) queued = false;
+    return err;
+  }
   void release() {
+    (void)settle();
     if (buf && pinned)
       (void)hipHostFree(buf);
     else
@@ -560,6 +570,7 @@ int run_set(hk_ggml_experts* set, const float* input, int input_rows, const int3
   auto* dy = reinterpret_cast<float*>(set->scratch.buf + in_bytes);
   if (int rc = set->stage.reserve(in_bytes + out_floats * sizeof(float))) return rc;
   pack_inputs(input, input_rows, (int)set->in, set->in, reinterpret_cast<uint16_t*>(set->stage.buf));
+  set->stage.queued = true;
   hipError_t err = hipMemcpyAsync(dx, set->stage.buf, (size_t)input_rows * set->ld * 2, hipMemcpyHostToDevice, nullptr);
   if (err != hipSuccess) return hip_fail(err, "expert input copy");
   auto* results = reinterpret_cast<float*>(set->stage.buf + in_bytes);
@@ -569,7 +580,7 @@ int run_set(hk_ggml_experts* set, const float* input, int input_rows, const int3
   set->last_slots = n;
   set->last_input_rows = input_rows;
   if (!set->stage.pinned) err = hipMemcpyAsync(results, dy, out_floats * sizeof(float), hipMemcpyDeviceToHost, nullptr);
-  if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
+  if (err == hipSuccess) err = set->stage.settle();
   if (err != hipSuccess) return hip_fail(err, "expert output copy");
   std::memcpy(out, results, out_floats * sizeof(float));
   return HK_OK;
@@ -865,6 +876,7 @@ uint16_t* coli_stage_inputs(const float* input, int rows, int cols, size_t extra
   if (rt.scratch.reserve(in_bytes + extra_bytes)) return nullptr;
   if (rt.stage.reserve(in_bytes + out_floats * sizeof(float))) return nullptr;
   pack_inputs(input, rows, cols, cols, reinterpret_cast<uint16_t*>(rt.stage.buf));
+  rt.stage.queued = true;
   if (hipMemcpyAsync(rt.scratch.buf, rt.stage.buf, copied, hipMemcpyHostToDevice, nullptr) != hipSuccess)
     return nullptr;
   *rest = rt.scratch.buf + in_bytes;
@@ -885,7 +897,7 @@ int coli_results(const float* dy, size_t n, float* output) {
   if (!rt.stage.pinned &&
       hipMemcpyAsync(results, dy, n * sizeof(float), hipMemcpyDeviceToHost, nullptr) != hipSuccess)
     return 0;
-  if (hipStreamSynchronize(nullptr) != hipSuccess) return 0;
+  if (rt.stage.settle() != hipSuccess) return 0;
   std::memcpy(output, results, n * sizeof(float));
   return 1;
 }
