@@ -35,7 +35,10 @@ int fail(const std::string& message) {
   return HK_ERR_INVALID;
 }
 
+// (HIP keeps a failed call's error for the next hipGetLastError, which would
+// be that of some later launch; it is reported here and no longer)
 int hip_fail(hipError_t err, const char* what) {
+  (void)hipGetLastError();
   set_error(std::string(what) + ": " + hipGetErrorString(err));
   return HK_ERR_HIP;
 }

@@ -36,7 +36,7 @@ struct Call {
 std::list<Pending> queue;
 std::map<char*, size_t> pinned;
 std::map<char*, size_t> device;
-long early_sources = 0, early_launches = 0, fail_in = -1, fail_malloc_of = -1;
+long early_sources = 0, early_launches = 0, fail_in = -1, fail_malloc_in = -1;
 hipError_t last = hipSuccess;
 
 hipError_t note(hipError_t err) {
@@ -77,8 +77,8 @@ long fake_early_sources() { return early_sources; }
 long fake_early_launches() { return early_launches; }
 // The launch after the next `n` fails; -1: none.
 void fake_fail_launch(long n) { fail_in = n; }
-// The next hipMalloc of at least `bytes` fails.
-void fake_fail_malloc(long bytes) { fail_malloc_of = bytes; }
+// The hipMalloc after the next `n` fails; -1: none.
+void fake_fail_malloc_after(long n) { fail_malloc_in = n; }
 // Bytes of device memory in use.
 long fake_device_bytes() {
   long n = 0;
@@ -102,10 +102,7 @@ hipError_t hipGetSymbolAddress(void** p, const void*) {
 
 hipError_t hipMalloc(void** p, size_t n) {
   *p = nullptr;
-  if (fail_malloc_of >= 0 && (long)n >= fail_malloc_of) {
-    fail_malloc_of = -1;
-    return note(hipErrorOutOfMemory);
-  }
+  if (fail_malloc_in >= 0 && fail_malloc_in-- == 0) return note(hipErrorOutOfMemory);
   *p = std::calloc(1, n ? n : 1);
   device[static_cast<char*>(*p)] = n;
   return hipSuccess;

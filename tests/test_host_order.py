@@ -102,3 +102,20 @@ for n in (64, 64, 256):
 matmul(256)
 settled()
 """)
+
+
+def test_expert_call_after_a_failed_reservation(child):
+    """A set whose scratch could not be had at its creation reserves it again
+    with a call, which then succeeds: the old failure is not reported again."""
+    child("""
+rng = np.random.default_rng(0)
+hip.init(0)
+w = rng.normal(size=(8, 64, 256)).astype(np.float32)
+x = rng.normal(size=(2, 256)).astype(np.float32)
+fake.fake_fail_malloc_after(2)  # (int8 rows and their scales first)
+s = GgmlExperts(w)
+s.mul_mat_id(x, [0, 1])
+fake.fake_fail_malloc_after(0)
+fails(lambda: GgmlExperts(w))
+s.mul_mat_id(x, [0, 1])
+""")
