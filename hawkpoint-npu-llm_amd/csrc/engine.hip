@@ -104,6 +104,7 @@ int op_scratch(OpScratch** out, size_t partial_floats, int counter_slots) {
     if (s.counters) HK_CHECK(hipFree(s.counters));
     HK_CHECK(hipMalloc(&s.counters, counter_slots * sizeof(unsigned int)));
     HK_CHECK(hipMemset(s.counters, 0, counter_slots * sizeof(unsigned int)));
+    HK_CHECK(hipStreamSynchronize(nullptr));  // (the caller's stream may be one that does not wait for the null stream)
     s.counter_slots = counter_slots;
   }
   s.device = dev;
@@ -615,6 +616,7 @@ int alloc_prefill_buffers(hk_engine* e, int rows) {
   const size_t slab_words = (size_t)((d.hidden + 15) / 16) * kSlabParts * kSlabMaxTokens * 16;
   HK_TRY(dalloc(&e->slab_ws, slab_words));
   HK_CHECK(hipMemset(e->slab_ws, 0, slab_words * sizeof(unsigned long long)));
+  HK_CHECK(hipStreamSynchronize(nullptr));  // (the engine's stream does not wait for the null stream)
   return 0;
 }
 

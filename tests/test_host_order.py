@@ -119,3 +119,19 @@ fake.fake_fail_malloc_after(0)
 fails(lambda: GgmlExperts(w))
 s.mul_mat_id(x, [0, 1])
 """)
+
+
+def test_first_prefill_waits_for_its_cleared_workspace(child):
+    """The workspace's tickets and tags are cleared on the null stream, which
+    the engine's stream does not wait for by itself."""
+    child("""
+e = engine()
+assert fake.fake_early_launches() == 0
+e.prefill(np.arange(70))
+assert fake.fake_early_launches() == 0, "kernels launched before the workspace was cleared"
+stream = ctypes.c_void_p()
+hip.check(hip.lib().hk_stream_create(ctypes.byref(stream)), "stream")
+b = [hip.DeviceBuffer(1 << 16) for _ in range(7)]
+hip.check(hip.lib().hk_attention_decode(*[x.ptr for x in b[:5]], 300, 512, 4, 2, 64, b[5].ptr, stream.value), "attention")
+assert fake.fake_early_launches() == 0, "attention launched before its tickets were cleared"
+""")
