@@ -676,12 +676,12 @@ int native_copies(hk_engine* e) {
 
 // The bf16 copies of a W8 engine's layer projections that the GEMMs of chunks
 // over kSlabMaxTokens read, one allocation made the first time such a chunk
-// runs (QKV and O come from the XCD split's copies where the engine has
-// them).  Without the memory for it the chunk runs on the int8 weights and a
-// later one tries again.
+// runs on the ring (QKV and O come from the XCD split's copies where the
+// engine has them).  Without the memory for it the chunk runs on the int8
+// weights and a later one tries again.
 int wide_copies(hk_engine* e) {
   const hk_model_desc& d = e->d;
-  if (!e->w8 || e->pf_wide != nullptr) return 0;
+  if (!e->w8 || e->pf_wide != nullptr || !prefill_ring_on()) return 0;
   const bool have = !e->wide.empty();
   const size_t nq = (size_t)e->qkv_rows * d.hidden, no = (size_t)d.hidden * d.q_heads * kHeadDim;
   const size_t ng = (size_t)2 * d.intermediate * d.hidden, nd = (size_t)d.hidden * d.intermediate;

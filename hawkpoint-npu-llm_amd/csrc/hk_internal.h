@@ -266,6 +266,9 @@ constexpr int kSlabNormMaxK = 1024;
 // compute units of the current device
 int cu_count();
 
+// Whether the GEMMs of more than 64 tokens may run on the LDS ring.
+bool prefill_ring_on();
+
 // float32 workspace the K-split path needs for an M x N residual GEMM with K
 // columns: one M x N slice per part (0 when the GEMM is not split).
 size_t split_ws_need(int M, int N, int K);

@@ -1524,6 +1524,16 @@ int ring_parts(int M, int N, int K) {
 }
 }  // namespace
 
+// HK_GEMM_RING=0 runs the GEMMs of more than 64 tokens on gemm_kernel instead
+// of gemm_ring_kernel (read once).
+bool prefill_ring_on() {
+  static const bool on = [] {
+    const char* v = std::getenv("HK_GEMM_RING");
+    return !(v && v[0] == '0');
+  }();
+  return on;
+}
+
 size_t split_ws_need(int M, int N, int K) {
   const int parts = ring_parts(M, N, K);
   return parts > 1 ? (size_t)parts * M * N : 0;
@@ -1582,16 +1592,6 @@ int launch_slab(const PrefillGemmArgs& a, hipStream_t stream) {
   return err == hipSuccess ? 0 : hip_fail(err, "slab gemm launch");
 }
 
-// HK_GEMM_RING=0 runs the GEMMs of more than 64 tokens on gemm_kernel instead
-// of gemm_ring_kernel (read once).
-bool ring_gemm() {
-  static const bool on = [] {
-    const char* v = std::getenv("HK_GEMM_RING");
-    return !(v && v[0] == '0');
-  }();
-  return on;
-}
-
 // Whether the ring takes a GEMM of more than 64 tokens: bf16 weights (W8: their
 // bf16 copy), operands whose bytes fit a buffer resource, and 16-byte rows for
 // its buffer -> LDS loads.
@@ -1599,7 +1599,7 @@ bool ring_takes(const PrefillGemmArgs& a) {
   const bool fits = (long long)a.M * a.lda * 2 < (1ll << 31) &&
                     (a.epi == EPI_SWIGLU ? 2ll : 1ll) * a.N * a.K * 2 < (1ll << 31);
   const uint16_t* w = a.scale ? a.Wx : a.W;
-  return w && ring_gemm() && a.M > kSlabMaxTokens && a.K % 32 == 0 && fits &&
+  return w && prefill_ring_on() && a.M > kSlabMaxTokens && a.K % 32 == 0 && fits &&
          ((reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;
 }
 

@@ -120,7 +120,16 @@ int hk_engine_generate(hk_engine* engine, int32_t token, int32_t position, int32
  * float32 summation order.  Replaces the reference's per-position prefill
  * loop (npu_llm/runtime/generate.py:1110-1125) and the engine's lm_head=False
  * dispatches (npu_llm/designs/qwen_engine.py:213-219).  Prompts longer than
- * 4096 tokens (or the context length) run in chunks of that many. */
+ * 4096 tokens (or the context length) run in chunks of that many.
+ * Device memory besides the model's: the first prompt allocates the row
+ * buffers, the first chunk of at most 64 tokens a copy of the layer
+ * projections in the order its GEMMs read (the same size again), and with
+ * HK_MODEL_W8 the first longer one a bf16 copy of them (two bytes per weight;
+ * for the models of the split decode step gate_up and down only, as that step
+ * holds bf16 QKV and O).  All stay with the engine until it is destroyed.
+ * A call that cannot have the first copy fails; one that cannot have the bf16
+ * copy runs on the int8 weights, slower, as all do with HK_GEMM_RING=0 in the
+ * environment. */
 int hk_engine_prefill(hk_engine* engine, const int32_t* tokens_host, int32_t n, int32_t start,
                       float* logits_host, int32_t* next_token_host);
 

@@ -135,3 +135,17 @@ b = [hip.DeviceBuffer(1 << 16) for _ in range(7)]
 hip.check(hip.lib().hk_attention_decode(*[x.ptr for x in b[:5]], 300, 512, 4, 2, 64, b[5].ptr, stream.value), "attention")
 assert fake.fake_early_launches() == 0, "attention launched before its tickets were cleared"
 """)
+
+
+@pytest.mark.parametrize("ring", ["1", "0"])
+def test_bf16_copies_only_where_the_ring_reads_them(child, ring):
+    """A W8 prompt of more than 64 tokens makes bf16 copies of the projections
+    for the ring GEMM; without the ring (HK_GEMM_RING=0) nothing reads them."""
+    child(f"""
+e = engine(w8=True)
+e.prefill(np.arange(40))
+before = fake.fake_device_bytes()
+e.prefill(np.arange(70), 40)
+per_layer = (2 + 2 * 1) * 64 * 128 + 128 * 128 + 3 * 256 * 128
+assert fake.fake_device_bytes() - before == ({ring} and 2 * 2 * per_layer), fake.fake_device_bytes() - before
+""", HK_GEMM_RING=ring)
