@@ -94,6 +94,12 @@ __device__ __forceinline__ u32x4 rotate8(const u32x4& own, const u32x4& other, c
   return o;
 }
 
+// 2^(score - max) with the maximum of a set of slots.  Where all of them score
+// -inf (a key with an infinite component) the maximum is no number to subtract:
+// they weigh 0 in the larger set they belong to, and only a row of nothing else
+// ends as 0 / 0, as the reference's softmax of it does.
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.0f : m; }
+
 __global__ __launch_bounds__(kThreads) void attention_decode_kernel(AttnArgs a) {
   const int p = a.position ? *a.position : a.pos;
   // workgroup b: chunk and head so that the heads of one chunk, which share
@@ -165,10 +171,11 @@ __global__ __launch_bounds__(kThreads) void attention_decode_kernel(AttnArgs a) 
       m = fmaxf(m, sc[i]);
     }
     m = groups_max(m);
+    const float m_use = finite_max(m);
     float sum = 0.0f, o[8] = {};
 #pragma unroll
     for (int i = 0; i < kRowsPerLane; ++i) {
-      const float e = __builtin_amdgcn_exp2f(sc[i] - m);
+      const float e = __builtin_amdgcn_exp2f(sc[i] - m_use);
       sum += e;
       const bool on = w0 + 8 * i + rg <= p;
 #pragma unroll
@@ -194,11 +201,12 @@ __global__ __launch_bounds__(kThreads) void attention_decode_kernel(AttnArgs a) 
   float m = wm[0];
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) m = fmaxf(m, wm[w]);
+  const float m_use = finite_max(m);
   float l = 0.0f, o = 0.0f;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
     if (t0 + 64 * w > p) break;
-    const float f = __builtin_amdgcn_exp2f(wm[w] - m);
+    const float f = __builtin_amdgcn_exp2f(wm[w] - m_use);
     l = fmaf(wl[w], f, l);
     o = fmaf(wo[w][lane], f, o);
   }
@@ -244,7 +252,7 @@ __global__ __launch_bounds__(kThreads) void attention_decode_kernel(AttnArgs a) 
   gm = wm[0];
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) gm = fmaxf(gm, wm[w]);
-  const float f = has ? __builtin_amdgcn_exp2f(cm - gm) : 0.0f;
+  const float f = has ? __builtin_amdgcn_exp2f(cm - finite_max(gm)) : 0.0f;
   weight[tid] = f;
   const float ls = group_sum<64>(has ? cl * f : 0.0f);
   if (lane == 0) wl[wave] = ls;

@@ -245,7 +245,7 @@ def test_argmax_first_maximum(hk_lib, n):
         assert int(_read(I, np.int32, 1)[0]) == int(np.argmax(x))
 
 
-def _attention_case(hk_lib, q_heads, kv_heads, ctx, position, seed):
+def _attention_case(hk_lib, q_heads, kv_heads, ctx, position, seed, infinite=(), sign=-1.0):
     from runtime import hip
     from runtime.qwen_engine import rope_tables
 
@@ -256,7 +256,13 @@ def _attention_case(hk_lib, q_heads, kv_heads, ctx, position, seed):
     vc = np.zeros((kv_heads, ctx, 64), np.uint16)
     kc[:, :position] = bf16.to_bits(rng.normal(0, 1, (kv_heads, position, 64)).astype(np.float32))
     vc[:, :position] = bf16.to_bits(rng.normal(0, 1, (kv_heads, position, 64)).astype(np.float32))
-    qkv_bits = bf16.to_bits(rng.normal(0, 1, (q_heads + 2 * kv_heads) * 64).astype(np.float32))
+    qkv = rng.normal(0, 1, (q_heads + 2 * kv_heads) * 64).astype(np.float32)
+    if infinite:  # scores of sign * inf at those slots: the angle of dimension 31 is next to nothing
+        q31 = qkv.reshape(-1, 64)[:q_heads, 31]
+        q31[:] = np.abs(q31) + 0.5
+        for lo, hi in infinite:
+            kc[:, lo:hi, 31] = bf16.to_bits(np.float32(sign * np.inf))
+    qkv_bits = bf16.to_bits(qkv)
     QKV, COS, SIN, KC, VC = _dev(qkv_bits), _dev(cos), _dev(sin), _dev(kc), _dev(vc)
     OUT = hip.DeviceBuffer(2 * q_heads * 64)
     hip.check(hk_lib.hk_attention_decode(QKV.ptr, COS.ptr, SIN.ptr, KC.ptr, VC.ptr, position, ctx,
@@ -295,3 +301,23 @@ def test_attention_decode_matches_oracle(hk_lib, q_heads, kv_heads, ctx, positio
     got = bf16.from_bits(out).astype(np.float64)
     assert np.all(np.abs(got - ref) <= _ulp(ref) + 1e-5)
     assert (out == bf16.to_bits(ref)).mean() >= 0.95
+
+
+@pytest.mark.parametrize(
+    "position,infinite,sign",
+    [(200, [(64, 128)], -1.0), (130, [(0, 128)], -1.0), (700, [(256, 512)], -1.0), (1100, [(0, 300), (512, 832)], -1.0),
+     (300, [(0, 300)], -1.0), (300, [(70, 71)], 1.0)],
+)
+def test_attention_decode_infinite_scores(hk_lib, position, infinite, sign):
+    """Scores of -inf weigh nothing, also where they are all that a wave (64
+    slots) or a chunk (256) has; one of +inf makes the head NaN, as NumPy's
+    softmax does."""
+    announce(f"attention p={position} infinite {infinite} {sign}")
+    with np.errstate(invalid="ignore"):
+        out, ref, *_ = _attention_case(hk_lib, 14, 2, 2048, position, position, infinite, sign)
+    got = bf16.from_bits(out).astype(np.float64)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    assert np.isnan(ref).all() if sign > 0 else np.isfinite(ref).all()
+    # (the bounds of test_attention_decode_matches_oracle)
+    ok = np.isfinite(ref)
+    assert np.all(np.abs(got - ref)[ok] <= _ulp(ref[ok]) + 1e-5)
