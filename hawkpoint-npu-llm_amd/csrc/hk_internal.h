@@ -241,8 +241,8 @@ struct PrefillGemmArgs {
   const void* Wn;
   // Long-K slab GEMM without RoPE, norm or SwiGLU only (the down
   // projection): with slab_ws, K is split kSlabParts ways over workgroups of
-  // one XCD.  Parts 1.. publish their float32
-  // partial sums as tagged words (slab_tag << 32 | bits) into slab_ws, which
+  // one XCD (slab_place.h).  Parts 1.. publish their float32 partial sums as
+  // tagged words (slab_tag << 32 | bits) into slab_ws, which
   // holds ceil(N / 16) * kSlabParts * kSlabMaxTokens * 16 of them; part 0
   // polls them from the XCD's L2, adds the parts in order and applies the
   // epilogue.  slab_tag is nonzero and new for every launch; a wait that

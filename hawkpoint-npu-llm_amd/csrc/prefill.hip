@@ -23,6 +23,7 @@
 
 #include "hk_common.h"
 #include "hk_internal.h"
+#include "slab_place.h"
 
 namespace hk {
 namespace {
@@ -770,18 +771,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_slab_kernel(PrefillGemmArgs a
   __shared__ float ssq[NORM ? kSlabWaves : 1][kSlabMaxTokens];
   __shared__ float inv_s[kSlabMaxTokens];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  // this workgroup's slab and K part: the KS parts of slab s are places
-  // s % 8 + 8 (KS (s / 8) + q), q = 0..KS-1, all on XCD s % 8: eight
-  // consecutive workgroups run on eight XCDs, from a start that depends on
-  // the hardware queue, and each takes the place of its eight that its XCD
-  // has (two on one XCD would leave a place empty: part 0's wait gives up)
+  // this workgroup's slab and K part (the parts of a slab share an XCD)
   int slab = blockIdx.x, part = 0;
   if constexpr (KS > 1) {
-    unsigned xcc;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-    const int r = blockIdx.x / 8;
-    part = r % KS;
-    slab = (int)(xcc & 7u) + 8 * (r / KS);
+    const SlabPlace place = slab_place((int)blockIdx.x, KS);
+    slab = place.slab, part = place.part;
     if (slab * 16 >= a.N) return;
   }
   const int n0 = slab * 16;
@@ -1557,7 +1551,7 @@ void launch_slab_nb(const PrefillGemmArgs& a, hipStream_t stream) {
   } else if constexpr (!PAIR) {
     // long K split kSlabParts ways inside an XCD, on 16 waves per part, when
     // every part can be resident at once (part 0 waits for the others)
-    const int split_grid = kSlabParts * 8 * ((slabs + 7) / 8);
+    const int split_grid = slab_places(slabs, kSlabParts);
     if (long_k && a.slab_ws && !a.rope.on && split_grid <= cu_count())
       hipLaunchKernelGGL((gemm_slab_kernel<false, false, W8, 16, NB, false, kSlabParts>), dim3(split_grid),
                          dim3(16 * 64), 0, stream, a);
