@@ -50,6 +50,7 @@ constexpr int kThreads = 256;
 constexpr int kMaxRouted = 64;   // one lane per routed expert
 constexpr int kMaxShared = 8;
 constexpr int kMaxTopK = 16;
+constexpr int kMaxWidth = 1 << 26;  // 16 rows of weights are one buffer resource (expert_slab)
 
 constexpr int kRouterRows = 16;  // routed experts per router_logits workgroup
 constexpr int kPlanThreads = 1024;
@@ -307,7 +308,7 @@ struct ExpertGemmArgs {
   const ExpertGroup* groups;  // gridDim.y entries
   const int32_t* a_rows;      // A row of each slot (PAIR; else the slot itself)
   long long w_stride;
-  int N, K, a_bytes;          // bytes of A
+  int N, K, a_bytes;          // bytes of A (PAIR)
 };
 
 // The outputs n0 .. of one group on RB blocks of 16 rows, NF weight fragments
@@ -321,23 +322,31 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   const int fr = lane & 15, fk = (lane >> 4) * 8;
   const int N = a.N, K = a.K;
   // Wn of an expert: [rows / 16][K / 8][16] pieces of 8 weights, so a
-  // fragment's 16 rows are one 256-byte run and a wave's K step one 1 KiB run
-  const __amdgpu_buffer_rsrc_t wr = rsrc(a.Wn + (size_t)g.expert * (size_t)a.w_stride, (PAIR ? 2 : 1) * N * K * 2);
-  const __amdgpu_buffer_rsrc_t ar = rsrc(a.A, a.a_bytes);
-  // this lane's piece of its weight row in each fragment, and the numbers of
-  // its A rows; outputs and rows past the ends read zero
-  constexpr unsigned kOutside = 0x7ffffff0u;
-  unsigned wofs[NF];
+  // fragment's 16 rows are one 256-byte run, a wave's K step one 1 KiB run and
+  // the 16 rows in all one run of 32 K bytes: a buffer resource each, so that
+  // no 32-bit size or offset spans the whole matrix (2 GiB and more from 2^29
+  // gate and up weights).  The same for the rows of A where they follow each
+  // other.  Steps, outputs and rows past the ends read zero.
+  const uint16_t* We = a.Wn + (size_t)g.expert * (size_t)a.w_stride;
+  __amdgpu_buffer_rsrc_t wr[NF], ar[PAIR ? 1 : RB];
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
-    const int n = n0 + 16 * (f % NO) + fr, r = f < NO ? n : N + n;
-    wofs[f] = n < N ? (unsigned)((((r >> 4) * (K >> 3) + (fk >> 3)) * 16 + (r & 15)) * 16) : kOutside;
+    const int n = n0 + 16 * (f % NO), r = f < NO ? n : N + n;
+    wr[f] = rsrc(We + (size_t)r * K, n < N ? 32 * K : 0);
   }
+  constexpr unsigned kOutside = 0x7ffffff0u;
+  const unsigned wofs = (unsigned)((fk >> 3) * 16 + fr) * 16u;  // this lane's piece of a fragment
   const __amdgpu_buffer_rsrc_t rr = rsrc(PAIR ? a.a_rows + g.offset : nullptr, PAIR ? g.rows * 4 : 0);
-  unsigned row[RB];
+  unsigned row[PAIR ? RB : 1];  // the numbers of this lane's A rows
+  if constexpr (PAIR) {
+    ar[0] = rsrc(a.A, a.a_bytes);
 #pragma unroll
-  for (int b = 0; b < RB; ++b)
-    row[b] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(rr, (16 * b + fr) * 4, 0, 0) : g.offset + 16 * b + fr;
+    for (int b = 0; b < RB; ++b) row[b] = __builtin_amdgcn_raw_buffer_load_b32(rr, (16 * b + fr) * 4, 0, 0);
+  } else {
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      ar[b] = rsrc(a.A + (size_t)(g.offset + 16 * b) * K, min(max(g.rows - 16 * b, 0), 16) * (2 * K));
+  }
   const int steps = K / 32;
   const int mine = steps > wave ? (steps - wave + WAVES - 1) / WAVES : 0;
   f32x4 acc[RB][NF];
@@ -349,18 +358,19 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   // loads of the step DEPTH on, so about DEPTH steps stay in flight (the
   // barriers keep the scheduler from pairing each load with its use)
   u32x4 w[DEPTH][NF], x[DEPTH][RB];
-  unsigned aofs[RB];
+  unsigned aofs[PAIR ? RB : 1];
   auto load_w = [&](int slot, int j) {
     const unsigned k0w = (unsigned)(wave + WAVES * j) * 1024u;  // four k groups of 16 pieces
 #pragma unroll
     for (int f = 0; f < NF; ++f)
-      w[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(wr, j < mine ? wofs[f] + k0w : kOutside, 0, 2);
+      w[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(wr[f], wofs + k0w, 0, 2);  // (past K: outside)
   };
   auto load_x = [&](int slot, int j) {
     const unsigned k0b = (unsigned)(wave + WAVES * j) * 64u;  // bytes along an A row
 #pragma unroll
     for (int b = 0; b < RB; ++b)
-      x[slot][b] = __builtin_amdgcn_raw_buffer_load_b128(ar, j < mine ? aofs[b] + k0b : kOutside, 0, 0);
+      x[slot][b] =
+          __builtin_amdgcn_raw_buffer_load_b128(ar[PAIR ? 0 : b], j < mine ? aofs[PAIR ? b : 0] + k0b : kOutside, 0, 0);
   };
   auto multiply = [&](int slot) {
 #pragma unroll
@@ -374,8 +384,12 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   for (int i = 0; i < DEPTH; ++i) load_w(i, i);
   __builtin_amdgcn_sched_barrier(0);
   // (after the weight loads: the rows' numbers are waited for here)
+  if constexpr (PAIR) {
 #pragma unroll
-  for (int b = 0; b < RB; ++b) aofs[b] = 16 * b + fr < g.rows ? (row[b] * (unsigned)K + fk) * 2u : kOutside;
+    for (int b = 0; b < RB; ++b) aofs[b] = 16 * b + fr < g.rows ? (row[b] * (unsigned)K + fk) * 2u : kOutside;
+  } else {
+    aofs[0] = (unsigned)(fr * K + fk) * 2u;
+  }
 #pragma unroll
   for (int i = 0; i < DEPTH; ++i) load_x(i, i);
   __builtin_amdgcn_sched_barrier(0);
@@ -503,10 +517,14 @@ int max_groups(const hk_moe_desc& d, int T) {
   return std::min(d.experts, pairs) + pairs / kGroupRows + d.shared * runs;
 }
 
+// Tokens whose rows one buffer resource spans (expert_slab's A rows are
+// gathered from all of them): a call of more runs in as many passes.
+int pass_tokens(const hk_moe_desc& d) { return std::max(1, 0x3ffffff0 / d.hidden); }
+
 // The expert GEMMs and the combine, after the plan.
 int moe_run(hk_moe* m, const uint16_t* x, int T, const float* weights, uint16_t* y, hipStream_t st) {
   const hk_moe_desc& d = m->d;
-  const int groups = max_groups(d, T), slots = T * (d.top_k + d.shared);
+  const int groups = max_groups(d, T);
   ExpertGemmArgs gu = {};
   gu.A = x;
   gu.Wn = m->gate_up_n;
@@ -526,7 +544,6 @@ int moe_run(hk_moe* m, const uint16_t* x, int T, const float* weights, uint16_t*
   dn.w_stride = (long long)d.hidden * d.intermediate;
   dn.N = d.hidden;
   dn.K = d.intermediate;
-  dn.a_bytes = slots * d.intermediate * 2;
   MOE_TRY(launch_expert_slab<false>(dn, groups, T >= kWideTokens, st));
   hipLaunchKernelGGL(combine_kernel, dim3(T, (d.hidden + kThreads - 1) / kThreads), dim3(kThreads), 0, st, m->out,
                      m->pair_slot, weights, d.hidden, d.top_k, d.shared, y);
@@ -540,6 +557,26 @@ int plan_route(hk_moe* m, const int32_t* ids, int T, hipStream_t st) {
                      max_groups(d, T), m->groups, m->a_rows, m->pair_slot);
   MOE_CHECK(hipGetLastError());
   return 0;
+}
+
+// The router, the top-k and the plan of T tokens.
+int route(hk_moe* m, const uint16_t* x, int T, int32_t* ids, float* weights, hipStream_t st) {
+  const hk_moe_desc& d = m->d;
+  hipLaunchKernelGGL(router_logits_kernel, dim3(T, (d.experts + kRouterRows - 1) / kRouterRows), dim3(kThreads), 0,
+                     st, x, m->router, d.hidden, d.experts, m->logits);
+  MOE_CHECK(hipGetLastError());
+  // one token per wave of the plan's workgroup, or the top-k spread over the
+  // GPU and the plan after it (one launch more)
+  if (T <= kPlanTokens) {
+    hipLaunchKernelGGL(topk_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, m->logits, T, d.experts, d.top_k,
+                       d.shared, max_groups(d, T), ids, weights, m->groups, m->a_rows, m->pair_slot);
+    MOE_CHECK(hipGetLastError());
+    return 0;
+  }
+  hipLaunchKernelGGL(topk_kernel, dim3((T + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0, st, m->logits,
+                     T, d.experts, d.top_k, ids, weights);
+  MOE_CHECK(hipGetLastError());
+  return plan_route(m, ids, T, st);
 }
 
 template <typename T>
@@ -562,6 +599,8 @@ int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_
   if (d.top_k <= 0 || d.top_k > d.experts || d.top_k > kMaxTopK) return fail("hk_moe_create: bad top_k");
   if (d.hidden <= 0 || d.hidden % 32 || d.intermediate <= 0 || d.intermediate % 32)
     return fail("hk_moe_create: hidden and intermediate must be positive multiples of 32");
+  if (d.hidden >= kMaxWidth || d.intermediate >= kMaxWidth)
+    return fail("hk_moe_create: hidden and intermediate must be below 2^26");
   if (d.max_tokens <= 0 || d.max_tokens > 256) return fail("hk_moe_create: max_tokens must be 1..256");
   hk_moe* m = new hk_moe();
   m->d = d;
@@ -607,22 +646,12 @@ int hk_moe_forward(hk_moe* m, const uint16_t* x, int32_t tokens, uint16_t* y, in
   if (tokens <= 0 || tokens > m->d.max_tokens) return fail("hk_moe_forward: token count out of range");
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const hk_moe_desc& d = m->d;
-  hipLaunchKernelGGL(router_logits_kernel, dim3(tokens, (d.experts + kRouterRows - 1) / kRouterRows),
-                     dim3(kThreads), 0, st, x, m->router, d.hidden, d.experts, m->logits);
-  MOE_CHECK(hipGetLastError());
-  // one token per wave of the plan's workgroup, or the top-k spread over the
-  // GPU and the plan after it (one launch more)
-  if (tokens <= kPlanTokens) {
-    hipLaunchKernelGGL(topk_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, m->logits, tokens, d.experts, d.top_k,
-                       d.shared, max_groups(d, tokens), m->ids, m->weights, m->groups, m->a_rows, m->pair_slot);
-    MOE_CHECK(hipGetLastError());
-  } else {
-    hipLaunchKernelGGL(topk_kernel, dim3((tokens + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0, st,
-                       m->logits, tokens, d.experts, d.top_k, m->ids, m->weights);
-    MOE_CHECK(hipGetLastError());
-    MOE_TRY(plan_route(m, m->ids, tokens, st));
+  for (int t0 = 0, T; t0 < tokens; t0 += T) {
+    T = std::min(tokens - t0, pass_tokens(d));
+    const size_t row = (size_t)t0 * d.hidden, pick = (size_t)t0 * d.top_k;
+    MOE_TRY(route(m, x + row, T, m->ids + pick, m->weights + pick, st));
+    MOE_TRY(moe_run(m, x + row, T, m->weights + pick, y + row, st));
   }
-  MOE_TRY(moe_run(m, x, tokens, m->weights, y, st));
   const size_t nk = (size_t)tokens * d.top_k;
   if (ids_out)
     MOE_CHECK(hipMemcpyAsync(ids_out, m->ids, nk * sizeof(int32_t), hipMemcpyDeviceToDevice, st));
@@ -643,8 +672,13 @@ int hk_moe_experts(hk_moe* m, const uint16_t* x, int32_t tokens, const int32_t* 
   MOE_CHECK(hipStreamSynchronize(st));
   for (int32_t e : host)
     if (e < 0 || e >= m->d.experts) return fail("hk_moe_experts: expert id out of range");
-  MOE_TRY(plan_route(m, ids, tokens, st));
-  return moe_run(m, x, tokens, weights, y, st);
+  for (int t0 = 0, T; t0 < tokens; t0 += T) {
+    T = std::min(tokens - t0, pass_tokens(m->d));
+    const size_t row = (size_t)t0 * m->d.hidden, pick = (size_t)t0 * m->d.top_k;
+    MOE_TRY(plan_route(m, ids + pick, T, st));
+    MOE_TRY(moe_run(m, x + row, T, weights + pick, y + row, st));
+  }
+  return 0;
 }
 
 void hk_moe_destroy(hk_moe* m) {

@@ -295,7 +295,9 @@ typedef struct hk_moe_desc {
 
 /* The block also makes an MFMA-native copy of every expert's gate/up and down
  * weights (the same size again, owned by the block, freed by hk_moe_destroy);
- * the caller's weights must stay unchanged while the block is used. */
+ * the caller's weights must stay unchanged while the block is used.  Hidden
+ * and intermediate sizes are multiples of 32 below 2^26; an expert's matrices
+ * may be of any size in bytes. */
 int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_t* gate_up,
                   const uint16_t* down, hk_moe** out);
 

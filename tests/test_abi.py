@@ -48,6 +48,17 @@ def test_error_path_without_gpu_work():
     assert "null" in hip.last_error()
 
 
+def test_moe_refuses_widths_its_kernels_do_not_span():
+    from runtime import hip
+    from runtime.moe import MoEDesc
+
+    lib, here, out = hip.lib(), ctypes.create_string_buffer(16), ctypes.c_void_p()
+    for hidden, intermediate in ((1 << 26, 32), (32, 1 << 26)):
+        desc = MoEDesc(hidden=hidden, intermediate=intermediate, experts=1, shared=0, top_k=1, max_tokens=1)
+        assert lib.hk_moe_create(ctypes.byref(desc), here, here, here, ctypes.byref(out)) == hip.HK_ERR_INVALID
+        assert "2^26" in hip.last_error()
+
+
 def _declared_experts():
     text = (ROOT / "include" / "hk_experts.h").read_text()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)

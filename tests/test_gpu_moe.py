@@ -170,6 +170,74 @@ def test_moe_row_groups_match_oracle(tokens, shape):
             assert rel_l2(bf16.from_bits(y3[t]), all_on(ids[0, 0], t)) <= 1e-2, t
 
 
+@pytest.mark.parametrize("hidden,intermediate,tokens",
+                         [(32768, 32800, 3), (32768, 32800, 40), ((1 << 23) + 32, 64, 130)])
+def test_moe_experts_of_more_than_2_gib(hk_lib, hidden, intermediate, tokens):
+    """Expert matrices and token rows that no 32-bit size spans: gate/up of
+    4 GiB per expert on few and many rows, and 2 GiB of token rows (two passes).
+    All zero but for the first and last hidden columns and intermediate rows, so
+    the oracle runs on those alone."""
+    import ctypes
+
+    from oracle.moe import expert_forward
+    from runtime import hip
+    from runtime.moe import MoEDesc
+
+    H, I, n = hidden, intermediate, 2  # one routed and one shared expert
+    announce(f"moe H={H} I={I} T={tokens}")
+    rng = np.random.default_rng(tokens)
+    bits = lambda *shape: bf16.to_bits(rng.normal(0, 0.3, shape).astype(np.float32))  # noqa: E731
+    columns, rows = (0, 32, H - 32), (0, 16, I - 16)  # two runs each: starts 0 and the last, their length between
+
+    def zeros(count):
+        b = hip.DeviceBuffer(2 * count)
+        b.zero()
+        return b
+
+    def runs(spec):
+        return [(spec[0], 0), (spec[2], spec[1])], spec[1]  # (start in the whole, start in the part), length
+
+    def place(buf, first, line, part, lines, spec):
+        """part's rows at the lines `lines` (each `line` long, from element `first`), in the runs of `spec`."""
+        starts, length = runs(spec)
+        for i, at in enumerate(lines):
+            for big, small in starts:
+                buf.write(part[i, small:small + length], 2 * (first + at * line + big))
+
+    def ends(spec):
+        starts, length = runs(spec)
+        return [big + i for big, _ in starts for i in range(length)]
+
+    x, gate_up, down = bits(tokens, 64), bits(n, 64, 64), bits(n, 64, 32)
+    bufs = dict(x=zeros(tokens * H), gate_up=zeros(n * 2 * I * H), down=zeros(n * H * I), y=zeros(tokens * H),
+                router=zeros(H))
+    place(bufs["x"], 0, H, x, range(tokens), columns)
+    for e in range(n):
+        inter = ends(rows)
+        place(bufs["gate_up"], e * 2 * I * H, H, gate_up[e], inter + [I + i for i in inter], columns)
+        place(bufs["down"], e * H * I, I, down[e], ends(columns), rows)
+    handle = ctypes.c_void_p()
+    desc = MoEDesc(hidden=H, intermediate=I, experts=1, shared=1, top_k=1, max_tokens=tokens)
+    try:
+        hip.check(hk_lib.hk_moe_create(ctypes.byref(desc), bufs["router"].ptr, bufs["gate_up"].ptr, bufs["down"].ptr,
+                                       ctypes.byref(handle)), "hk_moe_create")
+        hip.check(hk_lib.hk_moe_forward(handle.value, bufs["x"].ptr, tokens, bufs["y"].ptr, None, None, None), "moe")
+        hip.check(hk_lib.hk_stream_sync(None), "sync")
+        starts, length = runs(columns)
+        y = np.stack([np.concatenate([bufs["y"].read(np.uint16, length, 2 * (t * H + big)) for big, _ in starts])
+                      for t in range(tokens)])
+        middle = bufs["y"].read(np.uint16, 64, 2 * ((tokens - 1) * H + H // 2))
+    finally:
+        if handle.value:
+            hk_lib.hk_moe_destroy(handle.value)
+        for b in bufs.values():
+            b.free()
+    assert not middle.any()
+    for t in range(tokens):
+        ref = sum(expert_forward(gate_up[e], down[e], bf16.from_bits(x[t])) for e in range(n))
+        assert rel_l2(bf16.from_bits(y[t]), bf16.from_bits(bf16.to_bits(ref))) <= 1e-2, t
+
+
 def test_w8_expert_gemv_reference_pattern(hk_lib):
     """8 experts x 2048x2048 int8 with the reference test's pattern, scales and
     inputs; max error against the float-accumulated expectation < 0.03 (the
