@@ -488,8 +488,6 @@ struct hk_moe {
   std::mutex mu;
   hk_moe_desc d{};
   const uint16_t* router = nullptr;
-  const uint16_t* gate_up = nullptr;
-  const uint16_t* down = nullptr;
   uint16_t* gate_up_n = nullptr;  // MFMA-native copies of every expert (expert_slab_kernel)
   uint16_t* down_n = nullptr;
   float* logits = nullptr;       // [max_tokens * experts] router outputs
@@ -605,8 +603,6 @@ int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_
   hk_moe* m = new hk_moe();
   m->d = d;
   m->router = router;
-  m->gate_up = gate_up;
-  m->down = down;
   const size_t pairs = (size_t)d.max_tokens * (d.top_k + d.shared);
   const size_t groups = (size_t)d.experts + d.shared;
   auto body = [&]() -> int {

@@ -276,7 +276,7 @@ int hk_attention_decode_noalloc(const uint16_t* qkv, const float* rope_cos, cons
 int hk_stream_sync(void* stream);
 
 /* ---- routed-expert (MoE) block ----
- * Expert weights (device, bf16, caller-owned): router [E, H]; gate_up
+ * Weights (device, bf16, caller-owned): router [E, H]; gate_up
  * [E + S, 2 I, H] (gate rows then up rows); down [E + S, H, I].  Routed experts
  * are 0..E-1, the S shared experts follow.  Per token: r = router @ x (f32),
  * p = softmax(r), the top_k experts by p (ties to the lower id) weighted by p,
@@ -293,9 +293,10 @@ typedef struct hk_moe_desc {
   int32_t max_tokens;   /* largest batch, at most 256 */
 } hk_moe_desc;
 
-/* The block also makes an MFMA-native copy of every expert's gate/up and down
- * weights (the same size again, owned by the block, freed by hk_moe_destroy);
- * the caller's weights must stay unchanged while the block is used.  Hidden
+/* The block makes an MFMA-native copy of every expert's gate/up and down
+ * weights (the same size again, owned by the block, freed by hk_moe_destroy)
+ * before it returns and reads nothing but the copy from then on; the router
+ * stays the caller's and must not change while the block is used.  Hidden
  * and intermediate sizes are multiples of 32 below 2^26; an expert's matrices
  * may be of any size in bytes. */
 int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_t* gate_up,
