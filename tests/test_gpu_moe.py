@@ -170,6 +170,28 @@ def test_moe_row_groups_match_oracle(tokens, shape):
             assert rel_l2(bf16.from_bits(y3[t]), all_on(ids[0, 0], t)) <= 1e-2, t
 
 
+@pytest.mark.parametrize("tokens", [3, 20, 48, 150])
+def test_moe_rows_longer_than_the_ring(tokens):
+    """More K steps per wave than its ring holds, whole and partial last rounds,
+    on one, two and four 16-row blocks, narrow and wide."""
+    from runtime.moe import MoEBlock, synthetic_moe
+
+    H, I, E, K = 2336, 2080, 2, 2
+    announce(f"moe long rows T={tokens}")
+    router, gate_up, down = synthetic_moe(dict(hidden=H, intermediate=I, experts=E, shared=0), seed=4)
+    x = bf16.to_bits(np.random.default_rng(tokens).normal(0, 1, (tokens, H)).astype(np.float32))
+    b = MoEBlock(router, gate_up, down, top_k=K, shared=0, max_tokens=256)
+    try:
+        y, ids, w = b.forward(x)
+    finally:
+        b.close()
+    some = sorted({0, tokens // 2, tokens - 1})
+    ref_y, _, ref_w = moe_forward(x[some], router, gate_up, down, top_k=K, shared=0)
+    for i, t in enumerate(some):
+        np.testing.assert_allclose(w[t], ref_w[i], rtol=1e-5, atol=1e-7)
+        assert rel_l2(bf16.from_bits(y[t]), bf16.from_bits(ref_y[i])) <= 1e-2, t
+
+
 @pytest.mark.parametrize("hidden,intermediate,tokens",
                          [(32768, 32800, 3), (32768, 32800, 40), ((1 << 23) + 32, 64, 130)])
 def test_moe_experts_of_more_than_2_gib(hk_lib, hidden, intermediate, tokens):

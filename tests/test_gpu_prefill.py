@@ -145,7 +145,7 @@ def test_prefill_long_prompt():
     _prefill_case(model, _prompt(151936, 600, 14), 4, 1024, 1e-2, "qwen-2L-600")
 
 
-@pytest.mark.parametrize("shape,n", [("qwen", 65), ("qwen", 130), ("qwen", 417), ("qwen", 1021), ("smollm", 200),
+@pytest.mark.parametrize("shape,n", [("qwen", 65), ("qwen", 130), ("qwen", 350), ("qwen", 417), ("qwen", 1021), ("smollm", 200),
                                      ("wide", 65), ("wide", 300)])
 def test_prefill_between_slabs_and_long_prompts(shape, n):
     """65 to about a thousand tokens: the smaller tiles, the down projection
