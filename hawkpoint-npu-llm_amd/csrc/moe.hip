@@ -475,8 +475,13 @@ int launch_expert_slab(const ExpertGemmArgs& a, int groups, bool wide, hipStream
   return 0;
 }
 
-// Tokens from which the expert GEMMs run WIDE (expert_slab_kernel's figures:
-// even at 24 tokens, 4% of a call at 61).
+// Tokens from which the expert GEMMs run WIDE.  What decides is the rows per
+// expert and how many workgroups an expert makes; the line is in tokens, where
+// the 2048 / 64 + 2 x 1408 / top-6 block is even (24 to 32; 4% of a call at 61).
+// Narrow and wide elsewhere, us per call: 8 experts of 2048 x 4096, top-2, 4
+// tokens 64.7 and 61.4, 32 84.6 and 78.0; of 4096 x 7168, 8 tokens 142 and 154,
+// 24 218 and 220, 32 226 and 221; 64 of 2048 x 1408, top-1, 64 tokens 118 and
+// 124, 256 182 and 181.
 constexpr int kWideTokens = 33;
 
 }  // namespace

@@ -1499,15 +1499,23 @@ __global__ __launch_bounds__(kThreads * ST, ST == 1 ? 2 : 4) void attention_pref
 namespace {
 int tiles_of(int M, int N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// K parts of a residual GEMM on the ring's 64 x 64 tiles (1: no split): a
-// long K with too few tiles to fill the GPU is split over about one workgroup
-// per CU for the fewest tiles (their partial sums cost a pass each), two per
-// CU beyond, every part at least twelve 64-deep stages.  down_proj (K 4864,
-// N 896), us with the parts taken and unsplit or with one part fewer: 65
-// tokens 10.6 (6), 256 12.2 (4) and 13.4 (3), 417 15.0 (4) and 16.0 (3), 1021
-// 22.6 (2) and 23.2 (1).  A shorter K is split in two where that leaves the
-// RMSNorm after it to the second pass: O (K 896) and the norm, 100 tokens 7.4
-// against 6.9 + 3.5, 417 8.6 against 6.9 + 3.8, 1021 11.5 against 7.2 + 5.0.
+// K parts of a residual GEMM on the ring's 64 x 64 tiles (1: no split).  A long
+// K with too few tiles to fill the GPU is split: up to 64 tiles into about 256
+// workgroups (their partial sums cost a pass each), up to 224 into about 448,
+// a part about twelve 64-deep stages on average.  down_proj (K 4864, N 896: 14
+// tiles per 64 tokens), us with the parts taken and unsplit or with one part
+// fewer: 65 tokens 10.6 (6), 256 12.2 (4) and 13.4 (3), 417 15.0 (4) and 16.0
+// (3), 1021 22.6 (2) and 23.2 (1).  A shorter K is split in two where that
+// leaves the RMSNorm after it to the second pass: O (K 896) and the norm, 100
+// tokens 7.4 against 6.9 + 3.5, 417 8.6 against 6.9 + 3.8, 1021 11.5 against
+// 7.2 + 5.0.
+// The lines were drawn at what N 896 measured, not derived from the CU count.
+// Past 224 tiles (1024 tokens) O is better whole: four-layer prefills with O in
+// one part and in two, 1100 tokens 526 and 540 us, 1500 632 and 642, 2040 720
+// and 752.  Down in two or three would still be even or up to 2% of the prefill
+// faster (1100 tokens 529 whole, 525 in two; 1300 613, 608, 601 in three; 1500
+// 630, 620, 617; 1700 680, 677, 678) and loses at 2040 (727, 740).  N 576
+// (SmolLM2, K 576 and 1536): within 2% either way from 1021 to 1700 tokens.
 int ring_parts(int M, int N, int K) {
   const int t = tiles_of(M, N, 64, 64), stages = K / 64;
   if (t > 448 || N % 8 != 0) return 1;
@@ -1614,6 +1622,11 @@ void launch_ring_tiles(const PrefillGemmArgs& a, hipStream_t stream) {
 //   4064       17.0  15.9   -    62.7  64 x 128:  18.9  12.8   -   45.5
 // (before, on 128-token tiles with K split over a workspace pass: 12.0, 11.1,
 // 16.5 at 65 and 13.9, 13.3, 25.4 at 417.)
+// QKV with RoPE in its epilogue beyond that (24.0 us at 4064 on 128 x 128 tiles,
+// 32 deep): us per layer over that on 64 x 64, 64 x 128 and 128 x 64 tiles,
+// from four-layer prefills: 2300 tokens -1, 0, 3; 3000 2, 0, 3; 3600 -2, 4, 7;
+// 4064 -2.5, 4, 6.  (The table's figures are without RoPE, where 64 x 64 and
+// 64 x 128 look better.)
 //
 // W8: the bf16 copy of the int8 weights (every int8 value is a bf16 exactly)
 // with the row scales in the epilogue, the products and rounding points of the
