@@ -50,7 +50,7 @@ constexpr int kThreads = 256;
 constexpr int kMaxRouted = 64;   // one lane per routed expert
 constexpr int kMaxShared = 8;
 constexpr int kMaxTopK = 16;
-constexpr int kMaxWidth = 1 << 26;  // 16 rows of weights are one buffer resource (expert_slab)
+constexpr int kMaxWidth = 1 << 25;  // 64 rows of activations are one buffer resource (expert_slab)
 
 constexpr int kRouterRows = 16;  // routed experts per router_logits workgroup
 constexpr int kPlanThreads = 1024;
@@ -324,29 +324,26 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   // Wn of an expert: [rows / 16][K / 8][16] pieces of 8 weights, so a
   // fragment's 16 rows are one 256-byte run, a wave's K step one 1 KiB run and
   // the 16 rows in all one run of 32 K bytes: a buffer resource each, so that
-  // no 32-bit size or offset spans the whole matrix (2 GiB and more from 2^29
-  // gate and up weights).  The same for the rows of A where they follow each
-  // other.  Steps, outputs and rows past the ends read zero.
+  // no 32-bit size or offset spans the whole matrix (2 GiB and more from 2^30
+  // weights).  Where the rows of A follow each other, one resource over the
+  // group's (a resource per 16 rows: 233.1 us per 256-token call, so 231.8).
+  // Steps, outputs and rows past the ends read zero.
   const uint16_t* We = a.Wn + (size_t)g.expert * (size_t)a.w_stride;
-  __amdgpu_buffer_rsrc_t wr[NF], ar[PAIR ? 1 : RB];
+  __amdgpu_buffer_rsrc_t wr[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
     const int n = n0 + 16 * (f % NO), r = f < NO ? n : N + n;
     wr[f] = rsrc(We + (size_t)r * K, n < N ? 32 * K : 0);
   }
-  constexpr unsigned kOutside = 0x7ffffff0u;
+  constexpr unsigned kOutside = PAIR ? 0x7ffffff0u : 0xfffffff0u;  // past every resource of A
   const unsigned wofs = (unsigned)((fk >> 3) * 16 + fr) * 16u;  // this lane's piece of a fragment
   const __amdgpu_buffer_rsrc_t rr = rsrc(PAIR ? a.a_rows + g.offset : nullptr, PAIR ? g.rows * 4 : 0);
-  unsigned row[PAIR ? RB : 1];  // the numbers of this lane's A rows
-  if constexpr (PAIR) {
-    ar[0] = rsrc(a.A, a.a_bytes);
+  const __amdgpu_buffer_rsrc_t ar =
+      PAIR ? rsrc(a.A, a.a_bytes) : rsrc(a.A + (size_t)g.offset * K, (int)(2u * (unsigned)g.rows * (unsigned)K));
+  unsigned row[RB];  // the numbers of this lane's A rows in it
 #pragma unroll
-    for (int b = 0; b < RB; ++b) row[b] = __builtin_amdgcn_raw_buffer_load_b32(rr, (16 * b + fr) * 4, 0, 0);
-  } else {
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-      ar[b] = rsrc(a.A + (size_t)(g.offset + 16 * b) * K, min(max(g.rows - 16 * b, 0), 16) * (2 * K));
-  }
+  for (int b = 0; b < RB; ++b)
+    row[b] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(rr, (16 * b + fr) * 4, 0, 0) : 16 * b + fr;
   const int steps = K / 32;
   const int mine = steps > wave ? (steps - wave + WAVES - 1) / WAVES : 0;
   f32x4 acc[RB][NF];
@@ -358,7 +355,7 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   // loads of the step DEPTH on, so about DEPTH steps stay in flight (the
   // barriers keep the scheduler from pairing each load with its use)
   u32x4 w[DEPTH][NF], x[DEPTH][RB];
-  unsigned aofs[PAIR ? RB : 1];
+  unsigned aofs[RB];
   auto load_w = [&](int slot, int j) {
     const unsigned k0w = (unsigned)(wave + WAVES * j) * 1024u;  // four k groups of 16 pieces
 #pragma unroll
@@ -369,8 +366,7 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
     const unsigned k0b = (unsigned)(wave + WAVES * j) * 64u;  // bytes along an A row
 #pragma unroll
     for (int b = 0; b < RB; ++b)
-      x[slot][b] =
-          __builtin_amdgcn_raw_buffer_load_b128(ar[PAIR ? 0 : b], j < mine ? aofs[PAIR ? b : 0] + k0b : kOutside, 0, 0);
+      x[slot][b] = __builtin_amdgcn_raw_buffer_load_b128(ar, j < mine ? aofs[b] + k0b : kOutside, 0, 0);
   };
   auto multiply = [&](int slot) {
 #pragma unroll
@@ -384,12 +380,9 @@ __device__ __forceinline__ void expert_slab(const ExpertGemmArgs& a, const Exper
   for (int i = 0; i < DEPTH; ++i) load_w(i, i);
   __builtin_amdgcn_sched_barrier(0);
   // (after the weight loads: the rows' numbers are waited for here)
-  if constexpr (PAIR) {
 #pragma unroll
-    for (int b = 0; b < RB; ++b) aofs[b] = 16 * b + fr < g.rows ? (row[b] * (unsigned)K + fk) * 2u : kOutside;
-  } else {
-    aofs[0] = (unsigned)(fr * K + fk) * 2u;
-  }
+  for (int b = 0; b < RB; ++b)
+    aofs[b] = !PAIR || 16 * b + fr < g.rows ? (row[b] * (unsigned)K + fk) * 2u : kOutside;
 #pragma unroll
   for (int i = 0; i < DEPTH; ++i) load_x(i, i);
   __builtin_amdgcn_sched_barrier(0);
@@ -603,7 +596,7 @@ int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_
   if (d.hidden <= 0 || d.hidden % 32 || d.intermediate <= 0 || d.intermediate % 32)
     return fail("hk_moe_create: hidden and intermediate must be positive multiples of 32");
   if (d.hidden >= kMaxWidth || d.intermediate >= kMaxWidth)
-    return fail("hk_moe_create: hidden and intermediate must be below 2^26");
+    return fail("hk_moe_create: hidden and intermediate must be below 2^25");
   if (d.max_tokens <= 0 || d.max_tokens > 256) return fail("hk_moe_create: max_tokens must be 1..256");
   hk_moe* m = new hk_moe();
   m->d = d;

@@ -297,7 +297,7 @@ typedef struct hk_moe_desc {
  * weights (the same size again, owned by the block, freed by hk_moe_destroy)
  * before it returns and reads nothing but the copy from then on; the router
  * stays the caller's and must not change while the block is used.  Hidden
- * and intermediate sizes are multiples of 32 below 2^26; an expert's matrices
+ * and intermediate sizes are multiples of 32 below 2^25; an expert's matrices
  * may be of any size in bytes. */
 int hk_moe_create(const hk_moe_desc* desc, const uint16_t* router, const uint16_t* gate_up,
                   const uint16_t* down, hk_moe** out);

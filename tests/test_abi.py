@@ -53,10 +53,10 @@ def test_moe_refuses_widths_its_kernels_do_not_span():
     from runtime.moe import MoEDesc
 
     lib, here, out = hip.lib(), ctypes.create_string_buffer(16), ctypes.c_void_p()
-    for hidden, intermediate in ((1 << 26, 32), (32, 1 << 26)):
+    for hidden, intermediate in ((1 << 25, 32), (32, 1 << 25)):
         desc = MoEDesc(hidden=hidden, intermediate=intermediate, experts=1, shared=0, top_k=1, max_tokens=1)
         assert lib.hk_moe_create(ctypes.byref(desc), here, here, here, ctypes.byref(out)) == hip.HK_ERR_INVALID
-        assert "2^26" in hip.last_error()
+        assert "2^25" in hip.last_error()
 
 
 def _declared_experts():

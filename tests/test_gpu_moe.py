@@ -193,10 +193,11 @@ def test_moe_rows_longer_than_the_ring(tokens):
 
 
 @pytest.mark.parametrize("hidden,intermediate,tokens",
-                         [(32768, 32800, 3), (32768, 32800, 40), ((1 << 23) + 32, 64, 130)])
+                         [(32768, 32800, 3), (32768, 32800, 40), ((1 << 23) + 32, 64, 130), (64, (1 << 24) + 32, 70)])
 def test_moe_experts_of_more_than_2_gib(hk_lib, hidden, intermediate, tokens):
     """Expert matrices and token rows that no 32-bit size spans: gate/up of
-    4 GiB per expert on few and many rows, and 2 GiB of token rows (two passes).
+    4 GiB per expert on few and many rows, 2 GiB of token rows (two passes), and
+    of a group's intermediate rows.
     All zero but for the first and last hidden columns and intermediate rows, so
     the oracle runs on those alone."""
     import ctypes
@@ -248,7 +249,7 @@ def test_moe_experts_of_more_than_2_gib(hk_lib, hidden, intermediate, tokens):
         starts, length = runs(columns)
         y = np.stack([np.concatenate([bufs["y"].read(np.uint16, length, 2 * (t * H + big)) for big, _ in starts])
                       for t in range(tokens)])
-        middle = bufs["y"].read(np.uint16, 64, 2 * ((tokens - 1) * H + H // 2))
+        middle = bufs["y"].read(np.uint16, H - 64, 2 * ((tokens - 1) * H + 32))
     finally:
         if handle.value:
             hk_lib.hk_moe_destroy(handle.value)
