@@ -648,8 +648,8 @@ void free_native_copies(hk_engine* e) {
 // kSlabMaxTokens tokens), made the first time such a chunk runs: an engine
 // that only prefills long prompts never holds them.  Every matrix of an
 // engine shape has whole 16-row slabs (64-wide heads, hidden and
-// intermediate sizes multiples of 16).  On a failure every copy is freed, so
-// prefill_chunk then reads the row-major weights and a later chunk retries.
+// intermediate sizes multiples of 16).  On a failure every copy is freed and
+// the call fails; a later one starts over.
 int native_copies(hk_engine* e) {
   const hk_model_desc& d = e->d;
   if (!e->pf_native.empty() || d.hidden % 16 != 0 || d.intermediate % 16 != 0) return 0;
